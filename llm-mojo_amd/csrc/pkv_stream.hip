@@ -397,6 +397,7 @@ struct StreamArgs {
     int32_t nwg;       // P: workgroups along the keys
     int32_t nwg_cap;   // at most this many (the workspace holds nwg_cap + batch slots)
     int32_t lead;      // keys of split work charged to each sequence's start (set by the launcher)
+    int32_t weighted;  // stream_rows_kernel: keys weighted by their sequence's row tiles
     int32_t rows_seq;  // Hq * q_cnt: workspace rows per sequence
     int32_t* plan;     // [0] per_pair, [1] even, [2 + s] key prefix of sequence s (s <= batch)
     void* part_ml;     // Acc (m, l) per (slot, row)
@@ -476,6 +477,13 @@ __device__ inline KeySplit key_split(int total, int nwg) {
     return sp;
 }
 
+// Units of split work per key of a sequence with qc queries in this launch: what a key
+// costs stream_rows_kernel in matrix work and loads, by its 16-row tiles (one tile is bound
+// by its loads, two and three by the matrix cores).
+__device__ inline int row_units(const StreamArgs& a, int qc) {
+    return a.weighted ? 1 + 2 * ((a.G * qc + 15) >> 4) : 1;
+}
+
 // Exclusive scan of the key counts in s_pre[0..batch) (in place, one wave), total in
 // s_pre[batch].
 __device__ inline void wave_scan_counts(int* s_pre, int batch, int lane) {
@@ -506,7 +514,8 @@ __device__ inline void wave_scan_counts(int* s_pre, int batch, int lane) {
 // [batch + s] its query count in this launch, and with a fused append [2 batch + s] its
 // first appended row (tok_off[s]; [3 batch] = tok_off[batch]).
 // With a fused append, s_al (alloc_plan_ints(batch) ints) receives the allocation plan.
-template <int D, int ADDR>
+// WT: a sequence's keys count row_units() units each (stream_rows_kernel).
+template <int D, int ADDR, bool WT = false>
 __device__ inline KeySplit stream_setup(const StreamArgs& a, int* s_pre, int* s_lo, int* s_meta,
                                         int* s_al) {
     constexpr bool RING = ADDR == kAddrRing;
@@ -562,7 +571,8 @@ __device__ inline KeySplit stream_setup(const StreamArgs& a, int* s_pre, int* s_
                 lo = -2;
             }
         }
-        s_pre[i] = n > 0 ? n + a.lead : 0;
+        const int units = WT ? row_units(a, qc) : 1;
+        s_pre[i] = n > 0 ? n * units + a.lead : 0;
         s_lo[i] = lo;
         if (ADDR == kAddrPaged && fused) {
             const int len = a.nr.table_lens[i];
@@ -1863,6 +1873,481 @@ __global__ __launch_bounds__(kMaxWaves * kSW) void stream_mfma_kernel(StreamArgs
     }
 }
 
+// ---- fp64 MFMA path, 9..32 query rows per KV head: fp32 pools, head_dim 256 or 512 --------
+//
+// A verify of the engine's 5 tokens is 10 rows per kv head on the sliding layers and 40 on
+// the global ones; in groups of 8 rows it read the keys two and five times. Here one pass
+// over the keys serves up to 32 rows (RT tiles of 16). 16 sequences of 512..4096 keys, 1..5
+// tokens each: a ring layer of 16/8/256 84 -> 72 us with its merge, a global layer of 16/2/512
+// 304 -> 170 us (its fifth token is a second launch of the 8-row kernel), the two layers' whole
+// verify step 400 -> 250 us. What bounds it: the fp64 matrix rate, which fp64 vector work
+// (conversions, exponentials) shares -- a probe with one wave on each showed no overlap --
+// at 0.5-0.6 of it, the rest being waits at the batch's barrier and the pieces' starts.
+// Three tiles (40 rows) spilled; two batches of K in registers changed nothing.
+//
+// A workgroup is one kv head over one key range (the plan, pieces, partials and merge of the
+// kernels above), and its eight waves split the head's dims: wave v owns d in
+// [v DS, (v + 1) DS), DS = D / 8, of K, V, Q and O. Every K and V element is then used by one
+// wave only, in the lane it was loaded to, so K and V go from HBM straight into the registers
+// that feed v_mfma_f64_16x16x4 (no LDS staging, one conversion per element); against the
+// 4x4x4 kernel's row split an operand serves 16 rows instead of 4.
+// Lane L = i + 16 kk of v_mfma_f64_16x16x4 (checked on the device): A[i][kk], B[kk][i], and
+// register r of C holds C[kk + 4 r][i].
+//   S (16 tokens x 16 rows per tile): A = K (i = token), B = Q (i = row), k-step (c, e):
+//     d = v DS + 16 c + 4 kk + e. Each wave's S is a partial sum over its dims: the eight
+//     partials go through LDS (doubles) and are added by the wave that owns the row, one
+//     (row, token) per lane.
+//   Softmax there: one exponential per (row, token), the row's max only looked for when a
+//     score passes the lazy reference; P and the rows' rescale factors go back through LDS.
+//   O^T: A = V (i = d slot: d = v DS + VF i + e), B = P (kk = token, i = row).
+// One barrier per batch of T tokens: in the step of batch i a wave forms its partial scores
+// of batch i + 1, runs its softmax rows of batch i and the PV of batch i - 1 (S, P and the
+// factors are double-buffered). Waves 0-3 start with the softmax, waves 4-7 (the other wave
+// of each SIMD) end with it and take the matrix cores first (s_setprio: the arbiter would
+// favour the older wave; 110.7 -> 108.0 us and 72.6 -> 65.4 us below).
+// K of a batch is requested at least half a step, V a whole step before its use.
+// Every product of fp32 values is exact in double and every sum is a double sum, as in the
+// kernels above.
+// Tokens per batch: 64 KiB of K and V (32 KiB at head_dim 256 with two row tiles, whose S
+// would not fit in LDS otherwise).
+__host__ __device__ constexpr int rows_batch(int D, int rt) { return D == 512 || rt > 1 ? 16 : 32; }
+__host__ __device__ constexpr size_t rows_lds(int D, int batch, int rt) {
+    // per-sequence ints; two buffers each of the partial scores [8][16 rt][T + 2], P
+    // [16 rt][T + 2] and the factors [16 rt]
+    return mfma_stage_offset(batch, false) +
+           (size_t)2 * (9 * 16 * rt * (rows_batch(D, rt) + 2) + 16 * rt) * sizeof(double);
+}
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+typedef float f32x2v __attribute__((ext_vector_type(2)));
+typedef float f32x4v __attribute__((ext_vector_type(4)));
+
+template <int D, int RT, int ADDR>
+__global__ __launch_bounds__(kMaxWaves * kSW, 2) void stream_rows_kernel(StreamArgs a) {
+    constexpr bool RING = ADDR == kAddrRing;
+    constexpr bool PAGED = ADDR == kAddrPaged;
+    constexpr int NW = kMaxWaves;
+    constexpr int DS = D / NW;        // dims per wave
+    constexpr int T = rows_batch(D, RT);
+    constexpr int TT = T / 16;        // token tiles per batch
+    constexpr int TS = T / 4;         // PV steps per batch
+    constexpr int KC = DS / 16;       // float4 chunks of K (and Q) per lane and tile
+    constexpr int VF = DS / 16;       // d slots per lane and token of V: O tiles
+    constexpr int TP = T + 2;         // row stride of S and P in doubles (distinct banks)
+    constexpr int RPW = kSW / T;      // softmax rows per wave and round
+    constexpr int NP = (16 * RT + NW * RPW - 1) / (NW * RPW);  // softmax rounds
+    static_assert(NW == 8 && (VF == 2 || VF == 4), "eight waves over the dims");
+
+    extern __shared__ int smem[];
+    int* s_pre = smem;                         // [batch + 1]
+    int* s_lo = smem + a.batch + 1;            // [batch]
+    int* s_meta = smem + 2 * a.batch + 1;      // [3 batch + 1] (stream_setup)
+    double* const sS = reinterpret_cast<double*>(reinterpret_cast<char*>(smem) + mfma_stage_offset(a.batch, false));
+    double* const sP = sS + 2 * NW * 16 * RT * TP;
+    double* const sF = sP + 2 * 16 * RT * TP;
+
+    const int tid = threadIdx.x;
+    const int lane = tid & (kSW - 1);
+    const int wave = ufirst(tid / kSW);
+    const int w = blockIdx.x;
+    const int g = blockIdx.y;
+    const int B = a.batch;
+    const int i16 = lane & 15, kk = lane >> 4;
+    const KeySplit sp = stream_setup<D, ADDR, true>(a, s_pre, s_lo, s_meta, nullptr);
+    const int total = ufirst(s_pre[B]);
+    const int k0 = sp.start(w);
+    if (k0 >= total) return;
+    const int k1 = min(total, sp.start(w + 1));
+
+    const int rows = a.G * a.q_cnt;
+    const uint32_t row_bytes = (uint32_t)a.Hkv * D * 4;
+    const char* kbase = a.k_pool + ((size_t)g * D + wave * DS) * 4 + 16 * kk;
+    const char* vbase = a.v_pool + ((size_t)g * D + wave * DS + VF * i16) * 4;
+    const int bs_mask = (1 << a.bs_shift) - 1;
+    // this lane's score: row srow(p) of round p, token stok of the batch
+    const int stok = lane & (T - 1);
+    auto srow = [&](int p) { return (p * NW + wave) * RPW + lane / T; };
+
+    // barrier that waits for this wave's LDS accesses only: the K and V loads stay in flight
+    auto sync = [&]() {
+        __builtin_amdgcn_s_waitcnt(kLgkm0);
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+
+    int s = 0;
+    {
+        int lo = 0, hi = B - 1;
+        while (lo < hi) {
+            const int mid = (lo + hi + 1) >> 1;
+            if (ufirst(s_pre[mid]) <= k0) lo = mid;
+            else hi = mid - 1;
+        }
+        s = lo;
+    }
+    for (; s < B; ++s) {
+        const int ps = ufirst(s_pre[s]);
+        const int pe = ufirst(s_pre[s + 1]);
+        if (ps >= k1) break;
+        if (pe == ps) continue;
+        const int psr = ps + a.lead;
+        if (psr >= k1) break;
+        const int lo_key = ufirst(s_lo[s]);
+        const int pos0 = ufirst(s_meta[s]);
+        const int qc = ufirst(s_meta[B + s]);
+        const int rows_s = a.G * qc;
+        const int u = row_units(a, qc);
+        // A range of fewer units than a key's may hold no key: its piece is then empty.
+        const int ta = lo_key + (max(k0, psr) - psr + u - 1) / u;  // first key of the piece
+        const int tb = lo_key + (min(k1, pe) - psr + u - 1) / u;   // one past the last
+        const bool single = sp.owner(psr) == sp.owner(pe - 1);
+        const int32_t* trow = a.tables + (size_t)s * a.table_stride;
+        int64_t rbase = 0;  // ring mode: first row of the sequence's ring
+        int r0 = 0;         // ring mode: ring row of key ta
+        if constexpr (RING) {
+            rbase = a.pos ? (int64_t)ufirst(trow[0]) * a.ring_size : a.ring_base;
+            r0 = ta % a.ring_size;
+        }
+
+        // One body per number of live row tiles, so that no branch parts the MFMA chains.
+        auto piece = [&](auto NTc) {
+            constexpr int NT = decltype(NTc)::value;
+            bool bad = false;
+            bool left_out = false;  // a value at the edges that is not finite (see pv)
+            const int last = tb - 1;  // >= the sequence's first key, also in an empty piece
+            // Block table entry of this lane's token (lane mod T) of the batch at t.
+            auto entry = [&](int t) -> int {
+                if constexpr (PAGED) return trow[min(t + stok, last) >> a.bs_shift];
+                else return 0;
+            };
+            // Pool row of this lane's token of the batch at t; tokens past the piece re-read
+            // its last row and are masked.
+            auto pool_row = [&](int t, int ent) -> uint32_t {
+                const int tt = min(t + stok, last);
+                if constexpr (RING) return (uint32_t)ring_key_row(rbase, r0, max(tt - ta, 0), a.ring_size);
+                const bool id_ok = ent >= 0 && ent < a.num_blocks;
+                bad = bad || !id_ok;
+                return ((uint32_t)(id_ok ? ent : 0) << a.bs_shift) | (uint32_t)(tt & bs_mask);
+            };
+            f32x4v kf[TT][KC];
+            float vf[TS][VF];
+            auto load_k = [&](uint32_t prow) {
+#pragma unroll
+                for (int tt = 0; tt < TT; ++tt) {
+                    const uint32_t r = (uint32_t)__shfl((int)prow, 16 * tt + i16);
+                    const char* p = kbase + (size_t)r * row_bytes;
+#pragma unroll
+                    for (int c = 0; c < KC; ++c)
+                        kf[tt][c] = ld<true>(reinterpret_cast<const PKV_GLOBAL f32x4v*>((uintptr_t)(p + 64 * c)));
+                }
+            };
+            auto load_v = [&](uint32_t prow, int ts) {
+                const uint32_t r = (uint32_t)__shfl((int)prow, 4 * ts + kk);
+                const char* p = vbase + (size_t)r * row_bytes;
+                if constexpr (VF == 4) {
+                    const f32x4v v = ld<true>(reinterpret_cast<const PKV_GLOBAL f32x4v*>((uintptr_t)p));
+#pragma unroll
+                    for (int e = 0; e < VF; ++e) vf[ts][e] = v[e];
+                } else {
+                    const f32x2v v = ld<true>(reinterpret_cast<const PKV_GLOBAL f32x2v*>((uintptr_t)p));
+#pragma unroll
+                    for (int e = 0; e < VF; ++e) vf[ts][e] = v[e];
+                }
+            };
+            // The first batches' entries and the query rows share one round trip. Every load of
+            // the batch loop is issued, past the piece's end too (its last row again), so that no
+            // branch parts a load from its use and the waits stay exact.
+            const int ent0 = entry(ta);
+            int ent1 = entry(ta + T);
+            // Q: rows 16 rt + i16 of the head (rows past the last re-read it; masked)
+            f32x4v qf[NT][KC];
+#pragma unroll
+            for (int rt = 0; rt < NT; ++rt) {
+                const float* qp = a.q + out_row(a, s, g, min(16 * rt + i16, rows - 1)) * D + wave * DS + 4 * kk;
+#pragma unroll
+                for (int c = 0; c < KC; ++c) qf[rt][c] = *reinterpret_cast<const f32x4v*>(qp + 16 * c);
+            }
+            // pool rows of this lane's token in the batch whose V comes next and the one after
+            uint32_t row_v = pool_row(ta, ent0), row_k = row_v;
+            load_k(row_v);
+
+            f64x4 o[NT][VF];
+#pragma unroll
+            for (int rt = 0; rt < NT; ++rt)
+#pragma unroll
+                for (int e = 0; e < VF; ++e) o[rt][e] = f64x4{0, 0, 0, 0};
+            double m[NP], l[NP];
+#pragma unroll
+            for (int p = 0; p < NP; ++p) {
+                m[p] = -INFINITY;
+                l[p] = 0.0;
+            }
+            // key positions attended by every live row, and the tests of one row
+            const int pq_first = pos0 + a.j0, ws_last = window_start(pos0 + a.j0 + qc - 1, a.window);
+            auto attends = [&](int row, int tok) {
+                const int pq = pq_first + row / a.G;
+                return row < rows_s && tok < tb && tok <= pq && tok >= window_start(pq, a.window);
+            };
+
+            // The softmax rows of this wave of the batch at t: S, P and factors of buffer pb.
+            auto softmax = [&](int t, int pb) {
+#pragma unroll
+                for (int p = 0; p < NP; ++p) {
+                    const int row = srow(p);
+                    if ((p * NW + wave) * RPW >= 16 * NT) break;
+                    const double* ss = sS + (pb * NW * 16 * RT + row) * TP + stok;
+                    double v = 0.0;
+#pragma unroll
+                    for (int x = 0; x < NW; x += 2) v += ss[x * 16 * RT * TP] + ss[(x + 1) * 16 * RT * TP];
+                    v *= (double)a.scale;
+                    const bool ok = attends(row, t + stok);
+                    double f = 1.0;
+                    if (__any(ok && v > m[p] + (double)kLazyMove)) {  // m = -inf: any live key
+                        double mb = ok ? v : -INFINITY;
+                        mb = allreduce_rows<1, 1>(mb, OpMax());
+                        if constexpr (T == 32) {
+                            double x = mb, y = mb;
+                            swap_halves<16>(x, y);
+                            mb = fmax(x, y);
+                        }
+                        if (mb > m[p] + (double)kLazyMove) {
+                            f = exp_acc(m[p] - mb);  // m = -inf gives 0
+                            m[p] = mb;
+                        }
+                    }
+                    const double e = ok ? exp_acc(v - m[p]) : 0.0;
+                    l[p] = l[p] * f + e;
+                    sP[(pb * 16 * RT + row) * TP + stok] = e;
+                    if (stok == 0) sF[pb * 16 * RT + row] = f;
+                }
+            };
+            // PV of the batch at t with P and the factors of buffer pb; More: V of the next
+            // batch is requested as this one's is used up.
+            auto pv = [&](auto More, int t, int pb) {
+                double f[NT];
+                bool moved = false;
+#pragma unroll
+                for (int rt = 0; rt < NT; ++rt) {
+                    f[rt] = sF[pb * 16 * RT + 16 * rt + i16];
+                    moved = moved || f[rt] != 1.0;
+                }
+                if (t > ta && __any(moved)) {
+#pragma unroll
+                    for (int rt = 0; rt < NT; ++rt)
+#pragma unroll
+                        for (int e = 0; e < VF; ++e)
+#pragma unroll
+                            for (int r = 0; r < 4; ++r) o[rt][e][r] *= f[rt];
+                }
+                const double* pp = sP + (pb * 16 * RT + i16) * TP + kk;
+                // A key that some row masks meets that row's weight 0; a value that is not
+                // finite would still make 0 * inf = NaN there. Such values of the keys at the
+                // edges of the causal mask and the window (and of the rows read again past the
+                // piece's end) are left out here and added to their rows at the end.
+                if (t + T > min(pq_first + 1, tb) || t < ws_last) {
+#pragma unroll
+                    for (int ts = 0; ts < TS; ++ts) {
+                        const int tok = t + 4 * ts + kk;
+                        const bool edge = tok > pq_first || tok < ws_last || tok >= tb;
+#pragma unroll
+                        for (int e = 0; e < VF; ++e)
+                            if (edge && (__float_as_uint(vf[ts][e]) & 0x7f800000u) == 0x7f800000u) {
+                                vf[ts][e] = 0.f;
+                                left_out = left_out || tok < tb;
+                            }
+                    }
+                }
+#pragma unroll
+                for (int ts = 0; ts < TS; ++ts) {
+                    double pr[NT];
+#pragma unroll
+                    for (int rt = 0; rt < NT; ++rt) pr[rt] = pp[16 * rt * TP + 4 * ts];
+#pragma unroll
+                    for (int e = 0; e < VF; ++e) {
+                        const double vd = (double)vf[ts][e];
+#pragma unroll
+                        for (int rt = 0; rt < NT; ++rt)
+                            o[rt][e] = __builtin_amdgcn_mfma_f64_16x16x4f64(vd, pr[rt], o[rt][e], 0, 0, 0);
+                    }
+                    if constexpr (decltype(More)::value) load_v(row_v, ts);
+                }
+                // the accumulators stay ahead of the branches that follow
+#pragma unroll
+                for (int rt = 0; rt < NT; ++rt)
+#pragma unroll
+                    for (int e = 0; e < VF; ++e) asm volatile("" : "+v"(o[rt][e]));
+            };
+
+            // Partial scores (this wave's dims) of the batch at t into buffer pb. Q stays fp32 in
+            // registers and is converted at each use.
+            auto qk = [&](int t, int pb) {
+#pragma unroll
+                for (int rt = 0; rt < NT; ++rt)
+#pragma unroll
+                    for (int c = 0; c < KC; ++c) asm volatile("" : "+v"(qf[rt][c]));
+                f64x4 sc[TT][NT];
+#pragma unroll
+                for (int tt = 0; tt < TT; ++tt)
+#pragma unroll
+                    for (int rt = 0; rt < NT; ++rt) sc[tt][rt] = f64x4{0, 0, 0, 0};
+#pragma unroll
+                for (int c = 0; c < KC; ++c) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        double kd[TT];
+#pragma unroll
+                        for (int tt = 0; tt < TT; ++tt) kd[tt] = (double)kf[tt][c][e];
+#pragma unroll
+                        for (int rt = 0; rt < NT; ++rt) {
+                            const double qd = (double)qf[rt][c][e];
+#pragma unroll
+                            for (int tt = 0; tt < TT; ++tt)
+                                sc[tt][rt] = __builtin_amdgcn_mfma_f64_16x16x4f64(kd[tt], qd, sc[tt][rt], 0, 0, 0);
+                        }
+                    }
+                }
+                row_k = pool_row(t + T, ent1);  // K of the next batch, the entries of the one after
+                ent1 = entry(t + 2 * T);
+                load_k(row_k);
+#pragma unroll
+                for (int tt = 0; tt < TT; ++tt)
+#pragma unroll
+                    for (int rt = 0; rt < NT; ++rt) asm volatile("" : "+v"(sc[tt][rt]));
+#pragma unroll
+                for (int tt = 0; tt < TT; ++tt)
+#pragma unroll
+                    for (int rt = 0; rt < NT; ++rt)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r)
+                            sS[((pb * NW + wave) * 16 * RT + 16 * rt + i16) * TP + 16 * tt + kk + 4 * r] =
+                                sc[tt][rt][r];
+            };
+            const int nb = (tb - ta + T - 1) / T;
+            using Yes = std::true_type;
+            using No = std::false_type;
+            // Step of batch it (at t); the first has no PV, the last no scores to form.
+            auto step = [&](auto First, auto Last, int it, int t) {
+                const uint32_t row_vn = row_k;  // row of batch it + 1
+                if (wave >= NW / 2) __builtin_amdgcn_s_setprio(2);
+                else softmax(t, it & 1);
+                if constexpr (!decltype(Last)::value) qk(t + T, (it + 1) & 1);
+                if constexpr (!decltype(First)::value) {
+                    pv(Yes{}, t - T, (it - 1) & 1);
+                } else {
+#pragma unroll
+                    for (int ts = 0; ts < TS; ++ts) load_v(row_v, ts);
+                }
+                row_v = row_vn;
+                if (wave >= NW / 2) {
+                    __builtin_amdgcn_s_setprio(0);
+                    softmax(t, it & 1);
+                }
+                sync();
+            };
+            if (nb > 0) {
+                qk(ta, 0);
+                sync();
+                if (nb == 1) {
+                    step(Yes{}, Yes{}, 0, ta);
+                } else {
+                    step(Yes{}, No{}, 0, ta);
+                    int it = 1, t = ta + T;
+                    for (; it + 1 < nb; ++it, t += T) step(No{}, No{}, it, t);
+                    step(No{}, Yes{}, it, t);
+                }
+                pv(No{}, ta + (nb - 1) * T, (nb - 1) & 1);
+            }
+            bad = __any(bad);
+            if (__any(left_out)) {
+                for (int t = ta; t < tb; ++t) {
+                    if (t >= ws_last && t <= pq_first) continue;  // every row attends it
+                    size_t r;
+                    if constexpr (RING) {
+                        r = (size_t)ring_key_row(rbase, r0, t - ta, a.ring_size);
+                    } else {
+                        const int ent = trow[t >> a.bs_shift];
+                        r = ((size_t)(ent >= 0 && ent < a.num_blocks ? ent : 0) << a.bs_shift) | (size_t)(t & bs_mask);
+                    }
+                    const float* vr = reinterpret_cast<const float*>(a.v_pool + r * row_bytes) + (size_t)g * D +
+                                      wave * DS + VF * kk;
+#pragma unroll
+                    for (int rt = 0; rt < NT; ++rt)
+#pragma unroll
+                        for (int e = 0; e < VF; ++e)
+#pragma unroll
+                            for (int x = 0; x < 4; ++x) {
+                                const float v = vr[4 * VF * x + e];
+                                if ((__float_as_uint(v) & 0x7f800000u) == 0x7f800000u && attends(16 * rt + i16, t))
+                                    o[rt][e][x] += (double)v;
+                            }
+                }
+            }
+
+            // l of each row over its tokens, into the rows' owners
+#pragma unroll
+            for (int p = 0; p < NP; ++p) {
+                if ((p * NW + wave) * RPW >= 16 * NT) break;
+                const int row = srow(p);
+                double x = allreduce_rows<1, 1>(l[p], OpSum());
+                if constexpr (T == 32) {
+                    double y = x;
+                    swap_halves<16>(x, y);
+                    x += y;
+                }
+                if (stok == 0) {
+                    if (single) {
+                        sF[(nb & 1) * 16 * RT + row] = 1.0 / (x + 1e-10);  // the buffer PV no longer reads
+                    } else if (row < rows) {
+                        const int orow = (row / a.G) * a.Hq + g * a.G + row % a.G;
+                        double* pml = static_cast<double*>(a.part_ml) + ((size_t)(w + s) * a.rows_seq + orow) * 2;
+                        pml[0] = bad ? __builtin_nan("") : m[p];
+                        pml[1] = x;
+                    }
+                }
+            }
+            if (single) {
+                sync();
+#pragma unroll
+                for (int rt = 0; rt < NT; ++rt) {
+                    const int row = 16 * rt + i16;
+                    const double inv = sF[(nb & 1) * 16 * RT + row];
+                    if (row < rows_s) {
+                        float* op = a.out + out_row(a, s, g, row) * D + wave * DS + VF * kk;
+#pragma unroll
+                        for (int r = 0; r < 4; ++r)
+#pragma unroll
+                            for (int e = 0; e < VF; e += 2) {
+                                float2 v;
+                                v.x = bad ? __builtin_nanf("") : (float)(o[rt][e][r] * inv);
+                                v.y = bad ? __builtin_nanf("") : (float)(o[rt][e + 1][r] * inv);
+                                *reinterpret_cast<float2*>(op + 4 * VF * r + e) = v;
+                            }
+                    }
+                }
+                sync();  // the factors are read before the next piece's first batch writes them
+            } else {
+#pragma unroll
+                for (int rt = 0; rt < NT; ++rt) {
+                    const int row = 16 * rt + i16;
+                    if (row < rows) {
+                        const int orow = (row / a.G) * a.Hq + g * a.G + row % a.G;
+                        double* dst = static_cast<double*>(a.part_o) +
+                                      ((size_t)(w + s) * a.rows_seq + orow) * D + wave * DS + VF * kk;
+#pragma unroll
+                        for (int r = 0; r < 4; ++r)
+#pragma unroll
+                            for (int e = 0; e < VF; e += 2)
+                                *reinterpret_cast<double2*>(dst + 4 * VF * r + e) =
+                                    make_double2(o[rt][e][r], o[rt][e + 1][r]);
+                    }
+                }
+            }
+        };
+        const int nt = (rows_s + 15) >> 4;
+        if (RT == 1 || nt <= 1) piece(std::integral_constant<int, 1>{});
+        else piece(std::integral_constant<int, RT>{});
+    }
+}
+
 // ---- bf16 MFMA path: bf16 pools, head_dim 256, 5..8 query rows per KV head -------------
 //
 // One wave per KV head, up to 8 query rows (a 4-token verify at G = 2), batches of 16
@@ -2762,6 +3247,47 @@ int32_t launch_bf16_mfma(StreamArgs a, hipStream_t st) {
     return PKV_OK;
 }
 
+// fp32 pools with 9..32 query rows per kv head: stream_rows_kernel, grid (nwg, Hkv).
+#ifndef PKV_LEAD_ROWS
+#define PKV_LEAD_ROWS 64
+#endif
+constexpr int kRowsMax = 32;
+template <int D, int RT, int ADDR>
+int32_t launch_rows_kernel(StreamArgs a, hipStream_t st) {
+    const size_t lds = rows_lds(D, a.batch, RT);
+    const void* fn = reinterpret_cast<const void*>(&stream_rows_kernel<D, RT, ADDR>);
+    if (lds > 64 * 1024 && !reserve_lds(fn, (int)kStreamLdsMax))
+        return fail(PKV_ERR_HIP, "pkv_attend: could not reserve the kernel's LDS");
+    const int slots = fill_workgroups(fn, kMaxWaves * kSW, lds);
+    if (slots <= 0) return fail(PKV_ERR_HIP, "pkv_attend: occupancy query failed");
+    a.nwg = slots / a.Hkv > 0 ? slots / a.Hkv : 1;
+    if (a.nwg > a.nwg_cap) a.nwg = a.nwg_cap;
+    if (a.nwg > 1) a.nwg &= ~1;  // whole pairs (key_split)
+    // the weighted units of the split must fit an int
+    a.weighted = (int64_t)a.batch * (((int64_t)a.max_pos + 1) * 7 + PKV_LEAD_ROWS) <= INT32_MAX ? 1 : 0;
+    a.lead = PKV_LEAD_ROWS;
+    hipLaunchKernelGGL((stream_rows_kernel<D, RT, ADDR>), dim3(a.nwg, a.Hkv), dim3(kMaxWaves * kSW), lds, st, a);
+    if (hipGetLastError() != hipSuccess)
+        return fail(PKV_ERR_HIP, "pkv_attend: the attention launch failed");
+    hipLaunchKernelGGL((stream_merge_kernel<D, double>), dim3(a.rows_seq, a.batch), dim3(merge_threads<D>()), 0, st,
+                       a);
+    return PKV_OK;
+}
+template <int D, int RT>
+int32_t launch_rows_addr(StreamArgs a, hipStream_t st) {
+    return a.ring_size > 0 ? launch_rows_kernel<D, RT, kAddrRing>(a, st)
+                           : launch_rows_kernel<D, RT, kAddrPaged>(a, st);
+}
+template <int D>
+int32_t launch_many_rows(StreamArgs a, int rows, hipStream_t st) {
+    return rows <= 16 ? launch_rows_addr<D, 1>(a, st) : launch_rows_addr<D, 2>(a, st);
+}
+// Whether a launch of up to kRowsMax rows fits the CU's LDS at this batch.
+bool many_rows_fit(int D, int batch, int rows) {
+    const int rt = (rows + 15) >> 4;
+    return rows_lds(D, batch, rt) <= kStreamLdsMax;
+}
+
 template <int D, typename KV, int R, int WPH>
 int32_t launch_r(StreamArgs a, hipStream_t st) {
     if (a.keys) return launch_addr<D, KV, R, WPH, kAddrSparse>(a, st);
@@ -2878,12 +3404,24 @@ int32_t stream_attend(const pkv_params* p, const float* q, const void* k_pool,
     const bool bf16 = p->kv_dtype == PKV_DTYPE_BF16;
     // Queries in groups of at most 8 query rows per kv head, one launch pair each; the
     // launches share the workspace in stream order.
-    const int per_launch = 8 / G;
+    // fp32 pools: from 9 rows on, groups of up to kRowsMax rows, each one pass over the keys
+    // (10 rows 84 -> 72 us, 32 rows 251 -> 119 us against groups of 8; a remainder of up to 8
+    // rows keeps the 8-row kernels, which waste no matrix rows).
+    int per_launch = 8 / G;
+    if (!bf16 && G * q_len > 8) {
+        const int per = q_len < kRowsMax / G ? q_len : kRowsMax / G;
+        if (many_rows_fit(p->head_dim, batch, G * per)) per_launch = per;
+    }
     for (int j0 = 0; j0 < q_len; j0 += per_launch) {
         a.j0 = j0;
         a.q_cnt = q_len - j0 < per_launch ? q_len - j0 : per_launch;
         a.rows_seq = p->num_heads * a.q_cnt;
         const int rows = G * a.q_cnt;
+        if (rows > 8) {  // fp32 pools
+            const int32_t rc = p->head_dim == 256 ? launch_many_rows<256>(a, rows, st) : launch_many_rows<512>(a, rows, st);
+            if (rc != PKV_OK) return rc;
+            continue;
+        }
         const int32_t rc = bf16 ? launch_rows<uint16_t>(a, p->head_dim, rows, st)
                                 : launch_rows<float>(a, p->head_dim, rows, st);
         if (rc != PKV_OK) return rc;

@@ -1,0 +1,110 @@
+"""GPU parity of the 9..32-rows-per-kv-head attention launch (stream_rows_kernel, fp32 pools)
+against the oracle: row tiles (9, 16, 17, 32 rows, and one query group past 32), piece and
+batch edges (contexts 0 .. 33 and long ones, one sequence cut into many pieces), windows
+that open inside a batch, ring pools, and values that are not finite in keys some rows mask.
+Tolerances: tests/parity.py (sums in double, so 1e-5 against float64)."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+from pkv import F32, LayerSpec, hip, lib
+from pkv.engine import make_params
+from tests import parity
+from tests.test_gpu_attend import _batched_case
+
+pytestmark = pytest.mark.gpu
+
+EDGES = [0, 1, 14, 15, 16, 17, 31, 32, 33, 1500]
+
+
+@pytest.mark.parametrize("hq,hkv,d,q_len,window", [
+    (16, 8, 256, 5, 0), (16, 8, 256, 8, 20), (16, 8, 256, 9, 1024), (16, 8, 256, 16, 0),
+    (16, 8, 256, 17, 40), (12, 4, 256, 4, 0), (16, 2, 512, 2, 0), (16, 2, 512, 4, 0), (16, 2, 512, 3, 25),
+    (8, 8, 512, 9, 0), (16, 2, 512, 5, 1024),
+])
+def test_rows_match_oracle(gpu, hq, hkv, d, q_len, window):
+    print(f"[rows] {hq}q/{hkv}kv/{d} q_len={q_len} window={window}", flush=True)
+    rng = np.random.default_rng(hq + 31 * d + q_len)
+    _batched_case(rng, len(EDGES), q_len, np.array(EDGES), hq, hkv, d, 16, window, F32, 0.0625)
+
+
+@pytest.mark.parametrize("bs", [1, 4, 64])
+def test_rows_block_sizes(gpu, bs):
+    print(f"[rows] block size {bs}", flush=True)
+    rng = np.random.default_rng(bs)
+    _batched_case(rng, 3, 5, np.array([3, 130, 700]), 16, 8, 256, bs, 0, F32, 0.0625)
+
+
+def test_rows_one_long_sequence(gpu):
+    print("[rows] one sequence, 20000 keys over every workgroup", flush=True)
+    _batched_case(np.random.default_rng(5), 1, 4, np.array([20000]), 16, 2, 512, 16, 0, F32, 0.0625)
+
+
+def _call(name, p, q, k, v, tables, pos, q_lens=None, max_pos=None):
+    B, q_len, hq, d = q.shape
+    mp = int(pos.max()) + q_len - 1 if max_pos is None else max_pos
+    ws = hip.DeviceArray((lib.load().pkv_workspace_size(ctypes.byref(p), B, q_len, mp),), np.uint8)
+    a = [hip.DeviceArray.from_numpy(x) for x in (q, k, v, tables, pos)]
+    out = hip.DeviceArray((B, q_len, hq, d), np.float32, zero=True)
+    counts = [hip.DeviceArray.from_numpy(q_lens)] if q_lens is not None else []
+    lib.call(name, None, ctypes.byref(p), a[0].ptr, a[1].ptr, a[2].ptr, a[3].ptr, tables.shape[1], a[4].ptr,
+             *[c.ptr for c in counts], q_len, B, mp, out.ptr, ws.ptr, ws.nbytes)
+    return out.numpy()
+
+
+@pytest.mark.parametrize("hq,hkv,d,q_len", [(16, 8, 256, 5), (16, 8, 256, 9), (16, 2, 512, 4)])
+def test_rows_ring(gpu, hq, hkv, d, q_len):
+    # The same keys in a ring and in pages: the key split and every sum are the same.
+    print(f"[rows] ring {hq}q/{hkv}kv/{d} q_len={q_len}", flush=True)
+    rng = np.random.default_rng(q_len + d)
+    window, ring, bs, B = 200, 200 + 8, 16, 5
+    pos = np.array([0, 150, 203, 1000, 417], np.int32)
+    slots = rng.permutation(B).astype(np.int32)
+    nblk = (int(pos.max()) + q_len + bs - 1) // bs
+    tables = rng.permutation(B * nblk).astype(np.int32).reshape(B, nblk)
+    kv = rng.standard_normal((2, B, nblk * bs, hkv, d), dtype=np.float32)
+    paged = np.zeros((2, B * nblk, bs, hkv, d), np.float32)
+    rings = np.full((2, B, ring, hkv, d), np.nan, np.float32)
+    for s in range(B):
+        paged[:, tables[s]] = kv[:, s].reshape(2, nblk, bs, hkv, d)
+        for t in range(max(0, pos[s] + q_len - ring), pos[s] + q_len):
+            rings[:, slots[s], t % ring] = kv[:, s, t]
+    rings[np.isnan(rings)] = 7.0
+    q = rng.standard_normal((B, q_len, hq, d), dtype=np.float32)
+    pp = make_params(LayerSpec(hq, hkv, d, window, F32), bs, B * nblk, 0.0625)
+    pr = make_params(LayerSpec(hq, hkv, d, window, F32, ring), bs, B, 0.0625)
+    a = _call("pkv_attend", pp, q, paged[0], paged[1], tables, pos)
+    b = _call("pkv_attend", pr, q, rings[0], rings[1], slots.reshape(B, 1), pos)
+    assert np.array_equal(a, b)
+    lens = np.full(B, nblk, np.int32)
+    args = (q_len, hq, hkv, d, bs, window)
+    parity.check(a, O.attend(q, paged[0].ravel(), paged[1].ravel(), tables, lens, pos, *args, scale=0.0625),
+                 O.attend_f64(q, paged[0].ravel(), paged[1].ravel(), tables, pos, *args, scale=0.0625))
+
+
+@pytest.mark.parametrize("hq,hkv,d,q_len", [(16, 8, 256, 5), (16, 2, 512, 4)])
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan])
+def test_rows_masked_values_not_finite(gpu, hq, hkv, d, q_len, value):
+    # V of the last query's own key is not finite in dims 3 and d - 1: the rows
+    # before it mask that key and must not change; its own row carries the value.
+    print(f"[rows] {value} in a masked key, {hq}q/{hkv}kv/{d}", flush=True)
+    rng = np.random.default_rng(9)
+    bs, pos = 16, np.array([70, 29], np.int32)
+    nblk = 6
+    tables = rng.permutation(2 * nblk).astype(np.int32).reshape(2, nblk)
+    k = rng.standard_normal((2 * nblk, bs, hkv, d), dtype=np.float32)
+    v = rng.standard_normal((2 * nblk, bs, hkv, d), dtype=np.float32)
+    q = rng.standard_normal((2, q_len, hq, d), dtype=np.float32)
+    p = make_params(LayerSpec(hq, hkv, d, 0, F32), bs, 2 * nblk, 0.0625)
+    clean = _call("pkv_attend", p, q, k, v, tables, pos)
+    for s in range(2):
+        t = int(pos[s]) + q_len - 1
+        v[tables[s, t // bs], t % bs][:, [3, d - 1]] = value
+    got = _call("pkv_attend", p, q, k, v, tables, pos)
+    assert np.array_equal(got[:, :-1], clean[:, :-1])
+    last = got[:, -1]
+    assert np.array_equal(last[..., 4:d - 1], clean[:, -1][..., 4:d - 1])
+    want = np.full(last[..., [3, d - 1]].shape, value, np.float32)
+    assert np.array_equal(last[..., [3, d - 1]], want, equal_nan=True)
