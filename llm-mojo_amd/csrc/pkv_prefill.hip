@@ -533,6 +533,307 @@ __global__ __launch_bounds__(kNT) void prefill_kernel(PrefillArgs a) {
     }
 }
 
+// Short grids: too few 128-row workgroups to fill the chip (a few hundred chunk tokens of one
+// or two sequences). A workgroup takes 16 RT rows (16 RT / G queries of the G heads of one kv
+// head) and its eight waves share out the keys instead of the rows: wave v takes the 16-key
+// batches v, v + 8, ... and the waves' (m, l, O) are combined through LDS at the end. So the
+// launch has up to eight times the workgroups, each an eighth as long.
+//
+// Row r of the workgroup is query q0 + r / G of head g G + r % G. A wave stages its batch alone
+// (K and V of 16 keys, 16 KiB of LDS, the layout and swizzles of the tiles above), so the loop
+// has no barrier: wait for the copies, read the K operands (S^T for every row tile), then V's,
+// send the next batch's copies, softmax, PV.
+// PV takes P_hi and P_lo of the 16 keys in one v_mfma_f32_16x16x32_bf16: k = 8 grp + e is key
+// 4 grp + e % 4, P_hi for e < 4 and P_lo above, against V's operand of those keys given twice.
+// The row max is looked for across the lane groups only when a score passes the lazy
+// reference, the row sum only at the end.
+// One sequence of 333 tokens over 3001 cached ones (16q/8kv/256): 114 us in 48 workgroups of
+// 128 rows -> 62 us in 168 of 32; 64 tokens over 3000: 102 -> 41 us in 64 of 16. What bounds
+// it: every workgroup copies all its keys into LDS (128 KiB per round of 128 keys, 2048 cycles
+// at 64 B a cycle); a round takes about 3300 cycles with one tile and 4700 with two.
+template <int G, int RT>
+__global__ __launch_bounds__(kNT) void prefill_split_kernel(PrefillArgs a) {
+    constexpr int NW = kNT / 64;
+    constexpr int QB = 16 * RT / G;       // queries per workgroup
+    constexpr int kBT = 16;               // keys per batch
+    constexpr int kHalf = kBT * kD;       // elements of K (or V) of a batch
+    __shared__ __attribute__((aligned(512))) uint16_t sKV[NW][2 * kHalf];  // per wave: K, then V
+    __shared__ float sM[NW][16 * RT], sL[NW][16 * RT];
+    __shared__ int s_bad[NW];
+
+    // Workgroup order as in prefill_kernel.
+    const int lin = blockIdx.x;
+    const int pair = lin / a.Hkv;
+    const int g = (lin - pair * a.Hkv + (pair >> 3)) % a.Hkv;
+    const int s = pair / a.qtiles;
+    const int tile = a.qtiles - 1 - (pair - s * a.qtiles);
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int grp = lane >> 4;
+    const int l16 = lane & 15;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int row0 = a.q_off[s];
+    const int n_q = a.q_off[s + 1] - row0;
+    const int q0 = tile * QB;
+    const int pos0 = a.pos[s];
+    auto out_at = [&](int query, int h) -> float* {
+        return a.out + ((size_t)(row0 + query) * a.Hq + h) * kD;
+    };
+
+    // Contract violations, as in prefill_kernel.
+    const int hi_all = pos0 + n_q - 1;
+    const bool inactive = pos0 < 0;
+    const bool bad_seq = !inactive && n_q > 0 &&
+                         (hi_all > a.max_pos || (hi_all >> a.bs_shift) >= a.table_stride ||
+                          n_q > a.max_q);
+    if (tile == 0 && n_q > a.qtiles * QB && !inactive) {
+        for (int i = tid; i < (n_q - a.qtiles * QB) * G * kD; i += kNT) {
+            const int r = i / (G * kD), h = (i / kD) % G, d = i % kD;
+            out_at(a.qtiles * QB + r, g * G + h)[d] = __builtin_nanf("");
+        }
+    }
+    if (q0 >= n_q) return;
+    if (inactive || bad_seq) {
+        const float fill = inactive ? 0.f : __builtin_nanf("");
+        for (int i = tid; i < QB * G * kD; i += kNT) {
+            const int r = i / (G * kD), h = (i / kD) % G, d = i % kD;
+            if (q0 + r < n_q) out_at(q0 + r, g * G + h)[d] = fill;
+        }
+        return;
+    }
+
+    const int q_last = min(n_q, q0 + QB) - 1;
+    const int k_lo = window_start(pos0 + q0, a.window);
+    const int k_hi = pos0 + q_last;
+    const int min_qpos = pos0 + q0;                   // batches inside every row's range
+    const int max_ws = window_start(k_hi, a.window);  // need no mask
+    const int kb0 = k_lo & ~(kBT - 1);
+    const int32_t* trow = a.tables + (size_t)s * a.table_stride;
+    const int bs_mask = (1 << a.bs_shift) - 1;
+    const uint32_t row_bytes = (uint32_t)a.Hkv * kD * 2;
+    uint16_t* const sK = sKV[wave];
+    uint16_t* const sV = sKV[wave] + kHalf;
+
+    // Copies: instruction j (of eight) fills key rows 2j (lanes 0-31) and 2j + 1 of K, another
+    // those of V. The two keys lie in one block (block_size >= 8), whose table entry lane j
+    // holds.
+    // The lane's chunk of K in pair j is that of pair 0 with the bits of 2j flipped (the swizzle),
+    // V's likewise. These and the operand addresses below are formed from an opaque copy of the
+    // lane where they are used: kept in registers they would spill beside Q and O of two tiles.
+    auto opaque_lane = [&]() -> uint32_t {
+        uint32_t x = lane;
+        asm volatile("" : "+v"(x));
+        return x;
+    };
+    bool bad = false;
+    auto entry = [&](int t) { return trow[min(max(t + 2 * (lane & 7), k_lo), k_hi) >> a.bs_shift]; };
+    // Copies of K (Which 0) or V (1) of the batch at t, whose entries lanes 0-7 hold in ent.
+    auto issue = [&](auto Which, int t, int ent) {
+        constexpr int which = decltype(Which)::value;
+        const bool ok = (uint32_t)ent < (uint32_t)a.num_blocks;
+        bad = bad || !ok;
+        const int blk = ok ? ent : 0;
+        const uint32_t ln = opaque_lane(), hi = ln >> 5, p16 = ln & 31;
+        const uint32_t voff = hi * row_bytes + (which ? 16 * ((((p16 >> 1) ^ hi) << 1) | (p16 & 1)) : 16 * (p16 ^ hi));
+        const char* pool = reinterpret_cast<const char*>(which ? a.v_pool : a.k_pool) + (size_t)g * (kD * 2);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const uint32_t b = (uint32_t)__builtin_amdgcn_readlane(blk, j);
+            const uint64_t off = (uint64_t)((b << a.bs_shift) | (uint32_t)((t + 2 * j) & bs_mask)) * row_bytes;
+            copy16_to_lds(reinterpret_cast<const uint16_t*>(pool + off + (voff ^ ((which ? 64u : 32u) * j))),
+                          (which ? sV : sK) + 2 * j * kD);
+        }
+    };
+
+    const int t1 = kb0 + kBT * wave;  // this wave's first batch
+    constexpr int kStep = NW * kBT;
+    int ent = entry(t1);
+    // Q as the B operand of S^T: lane holds Q[row 16 rt + l16][32c + 8 grp .. +7]
+    bf16x8 qreg[RT][8];
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+        const int r = 16 * rt + l16, qi = min(q0 + r / G, n_q - 1);
+        const uint16_t* qp = a.q + ((size_t)(row0 + qi) * a.Hq + g * G + r % G) * kD + 8 * grp;
+#pragma unroll
+        for (int c = 0; c < 8; ++c) qreg[rt][c] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(qp + 32 * c));
+    }
+    if (t1 <= k_hi) {
+        issue(Par<0>{}, t1, ent);
+        issue(Par<1>{}, t1, ent);
+        ent = entry(t1 + kStep);
+    }
+
+    f32x4 o[RT][16];  // O^T: d-tile u holds dims 16u + 4 grp + r of this lane's row
+    float m[RT], l[RT];
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+        m[rt] = -INFINITY;
+        l[rt] = 0.f;
+#pragma unroll
+        for (int u = 0; u < 16; ++u) o[rt][u] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    // K operand of 32-dim step c: key l16, chunk (4c + grp) ^ l16. V operand of d-tile u: key
+    // z = 4 grp + l16 / 4, byte 512 z + 32 (u ^ z) + 8 (l16 & 3). (Rows of 512 bytes in an area
+    // aligned to 512: c and u flip address bits.)
+    for (int t = t1; t <= k_hi; t += kStep) {
+        asm volatile("s_waitcnt vmcnt(0)" : "+v"(ent) : : "memory");  // the batch is in LDS
+        if (t + kBT - 1 > k_hi) {
+            // Rows past the range's last key may hold anything: V's are zeroed, so that a value
+            // that is not finite cannot meet a zero weight.
+            for (int r = k_hi + 1 - t; r < kBT; ++r)
+                if (lane < 32) *reinterpret_cast<uint4*>(sV + r * kD + 8 * lane) = make_uint4(0, 0, 0, 0);
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        }
+        f32x4 st[RT];
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) st[rt] = f32x4{0.f, 0.f, 0.f, 0.f};
+        const uint32_t lk = opaque_lane(), ki = lk & 15;
+        const uint32_t kl = lds_addr(sK) + 512 * ki + 16 * ((lk >> 4) ^ (ki & 3)) + 64 * (ki >> 2);
+        // K's operands, all requested at once (one row tile) or in two halves (registers)
+        constexpr int KH = 8 / RT;
+        static_for<0, RT>([&](auto H) {
+            constexpr int c0 = decltype(H)::value * KH;
+            i32x4 ka[KH];
+            static_for<0, KH>([&](auto C) {
+                constexpr int c = c0 + decltype(C)::value;
+                ka[c - c0] = lds_read_b128<256 * (c >> 2)>(kl ^ (64u * (c & 3)));
+            });
+            static_for<0, KH>([&](auto C) {
+                constexpr int c = decltype(C)::value;
+                lgkm_wait<KH - 1 - c>(ka[c]);
+#pragma unroll
+                for (int rt = 0; rt < RT; ++rt)
+                    st[rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, ka[c]), qreg[rt][c0 + c],
+                                                                     st[rt], 0, 0, 0);
+            });
+        });
+        // V's operands, all at once (one row tile) or in two halves (two tiles: registers)
+        constexpr int VH = 16 / RT;
+        i32x2 vr[VH];
+        auto read_v = [&](auto H) {
+            constexpr int u0 = decltype(H)::value * VH;
+            const uint32_t lv = opaque_lane(), z = 4 * (lv >> 4) + ((lv & 15) >> 2);
+            const uint32_t v0 = lds_addr(sV) + 512 * z + 32 * z + 8 * (lv & 3);
+#pragma unroll
+            for (int u = 0; u < VH; ++u) vr[u] = lds_read_tr16<0>(v0 ^ (32u * (u0 + u)));
+            asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(vr[0]), "+v"(vr[1]), "+v"(vr[2]), "+v"(vr[3]));
+#pragma unroll
+            for (int u = 4; u < VH; ++u) asm volatile("" : "+v"(vr[u]));
+        };
+        const bool more = t + kStep <= k_hi;
+        const int ent_cur = ent;
+        if (more) issue(Par<0>{}, t + kStep, ent_cur);  // K has been read
+        read_v(Par<0>{});
+        if (RT == 1 && more) issue(Par<1>{}, t + kStep, ent_cur);
+        if (more) ent = entry(t + 2 * kStep);
+
+        const bool edge = t + kBT - 1 > min_qpos || t < max_ws;
+        bf16x8 pb[RT];
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+            float sv[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) sv[r] = st[rt][r] * a.scale_log2;
+            if (edge) {
+                const int qpos = pos0 + min(q0 + (16 * rt + l16) / G, n_q - 1);
+                const int ws_row = window_start(qpos, a.window);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int key = t + 4 * grp + r;
+                    sv[r] = key <= qpos && key >= ws_row ? sv[r] : -INFINITY;
+                }
+            }
+            const float mx = fmaxf(fmaxf(sv[0], sv[1]), fmaxf(sv[2], sv[3]));
+            if (__any(mx > m[rt] + 8.f)) {  // lazy reference (log2 units): p <= 256
+                const float row_mx = swap32_max(swap16_max(mx));
+                if (row_mx > m[rt] + 8.f) {
+                    const float alpha = exp2f(m[rt] - row_mx);  // m = -inf gives 0
+                    m[rt] = row_mx;
+                    l[rt] *= alpha;
+#pragma unroll
+                    for (int u = 0; u < 16; ++u) o[rt][u] *= alpha;
+                }
+            }
+            const float mu = m[rt] == -INFINITY ? 0.f : m[rt];
+            float p[4];
+            uint32_t hi[4], lo[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                p[r] = exp2f(sv[r] - mu);  // masked: exp2(-inf) = 0
+                hi[r] = __float_as_uint(p[r]) & 0xffff0000u;  // P_hi: p truncated to bf16
+                const uint32_t x = __float_as_uint(p[r] - __uint_as_float(hi[r]));
+                lo[r] = (x + 0x7FFFu + ((x >> 16) & 1u)) >> 16;  // the remainder, to nearest even
+            }
+            l[rt] += (p[0] + p[1]) + (p[2] + p[3]);
+            const i32x4 pk = {(int)((hi[0] >> 16) | hi[1]), (int)((hi[2] >> 16) | hi[3]),
+                              (int)(lo[0] | (lo[1] << 16)), (int)(lo[2] | (lo[3] << 16))};
+            pb[rt] = __builtin_bit_cast(bf16x8, pk);
+        }
+        auto pv = [&](auto H) {
+            constexpr int u0 = decltype(H)::value * VH;
+#pragma unroll
+            for (int u = 0; u < VH; ++u) {
+                const i32x4 va = {vr[u][0], vr[u][1], vr[u][0], vr[u][1]};
+#pragma unroll
+                for (int rt = 0; rt < RT; ++rt)
+                    o[rt][u0 + u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, va), pb[rt], o[rt][u0 + u], 0, 0, 0);
+            }
+        };
+        pv(Par<0>{});
+        if constexpr (RT > 1) {
+            read_v(Par<1>{});
+            if (more) issue(Par<1>{}, t + kStep, ent_cur);
+            pv(Par<1>{});
+        }
+    }
+    __builtin_amdgcn_s_waitcnt(0);
+
+    // The waves' rows: common max, rescaled sums, then wave v adds d-tiles 2v and 2v + 1.
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+        if (grp == 0) sM[wave][16 * rt + l16] = m[rt];
+    bad = __any(bad);
+    if (lane == 0) s_bad[wave] = bad ? 1 : 0;
+    __syncthreads();
+    bool any_bad = false;
+#pragma unroll
+    for (int v = 0; v < NW; ++v) any_bad = any_bad || s_bad[v] != 0;
+    float* const red = reinterpret_cast<float*>(&sKV[0][0]);  // [wave][d-tile][lane][4], 128 KiB
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+        float M = -INFINITY;
+#pragma unroll
+        for (int v = 0; v < NW; ++v) M = fmaxf(M, sM[v][16 * rt + l16]);
+        const float f = m[rt] == -INFINITY ? 0.f : exp2f(m[rt] - M);
+        const float lr = swap32_sum(swap16_sum(l[rt])) * f;
+        if (grp == 0) sL[wave][16 * rt + l16] = lr;
+        if (rt > 0) __syncthreads();  // the tile before has been added
+#pragma unroll
+        for (int u = 0; u < 16; ++u) *reinterpret_cast<f32x4*>(red + ((wave * 16 + u) * 64 + lane) * 4) = o[rt][u] * f;
+        __syncthreads();
+        float L = 0.f;
+#pragma unroll
+        for (int v = 0; v < NW; ++v) L += sL[v][16 * rt + l16];
+        const float inv = 1.f / (L + 1e-10f);
+        const int r = 16 * rt + l16, qi = q0 + r / G;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int u = 2 * wave + h;
+            f32x4 x = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int v = 0; v < NW; ++v) x += *reinterpret_cast<const f32x4*>(red + ((v * 16 + u) * 64 + lane) * 4);
+            if (qi < n_q) {
+                float4 y;
+                y.x = any_bad ? __builtin_nanf("") : x[0] * inv;
+                y.y = any_bad ? __builtin_nanf("") : x[1] * inv;
+                y.z = any_bad ? __builtin_nanf("") : x[2] * inv;
+                y.w = any_bad ? __builtin_nanf("") : x[3] * inv;
+                *reinterpret_cast<float4*>(out_at(qi, g * G + r % G) + 16 * u + 4 * grp) = y;
+            }
+        }
+    }
+}
+
 }  // namespace
 }  // namespace pkv
 
@@ -585,14 +886,39 @@ int32_t pkv_prefill(void* stream, const pkv_params* p, const void* q, const void
     a.max_q = max_q;
     a.max_pos = max_pos;
     a.out = out;
-    const int qb = 128 / G;
-    a.qtiles = (max_q + qb - 1) / qb;
+    // Query rows per workgroup: 16 or 32 (prefill_split_kernel) where that many workgroups all
+    // run at once, else 128. A round of resident workgroups over 1000 keys takes about 12.5 us
+    // with 16 rows, 20 us with 32 and 35 us with 128, so a second round of the smaller tiles
+    // never pays against one of the next (16q/8kv/256, 3000 cached tokens, one sequence:
+    // 256 new tokens 111.8 (128 rows) / 66.6 (32) / 49.9 us (16); 512: 123.5 / 76.6 / 99.6;
+    // 1024: 147.6 / 155.6 / 215.3).
+    const void* split_fn = G == 1   ? reinterpret_cast<const void*>(&prefill_split_kernel<1, 2>)
+                           : G == 2 ? reinterpret_cast<const void*>(&prefill_split_kernel<2, 2>)
+                                    : reinterpret_cast<const void*>(&prefill_split_kernel<4, 2>);
+    const int resident = device_fill_workgroups(split_fn, kNT, 0, INT32_MAX);
+    if (resident <= 0) return fail(PKV_ERR_HIP, "pkv_prefill: occupancy query failed");
+    auto workgroups = [&](int64_t r) { return ((int64_t)max_q * G + r - 1) / r * p->num_kv_heads * batch; };
+    const int rows = workgroups(16) <= resident ? 16 : (workgroups(32) <= resident ? 32 : 128);
+    const int qb = rows / G;
+    a.qtiles = (int)(((int64_t)max_q + qb - 1) / qb);
     // one workgroup id per (sequence, tile, kv head); the launch's work-items must fit in 32 bits
     const int64_t wgs = (int64_t)a.qtiles * p->num_kv_heads * batch;
     if (wgs > (int64_t)(UINT32_MAX / kNT))
         return fail(PKV_ERR_UNSUPPORTED, "pkv_prefill: too many (sequence, query tile, kv head) workgroups");
     const dim3 grid((uint32_t)wgs);
     hipStream_t st = static_cast<hipStream_t>(stream);
+    if (rows < 128) {
+        if (rows == 16) {
+            if (G == 1) hipLaunchKernelGGL((prefill_split_kernel<1, 1>), grid, dim3(kNT), 0, st, a);
+            else if (G == 2) hipLaunchKernelGGL((prefill_split_kernel<2, 1>), grid, dim3(kNT), 0, st, a);
+            else hipLaunchKernelGGL((prefill_split_kernel<4, 1>), grid, dim3(kNT), 0, st, a);
+        } else {
+            if (G == 1) hipLaunchKernelGGL((prefill_split_kernel<1, 2>), grid, dim3(kNT), 0, st, a);
+            else if (G == 2) hipLaunchKernelGGL((prefill_split_kernel<2, 2>), grid, dim3(kNT), 0, st, a);
+            else hipLaunchKernelGGL((prefill_split_kernel<4, 2>), grid, dim3(kNT), 0, st, a);
+        }
+        return check_launch("pkv_prefill");
+    }
     // The kernel's four 32 KiB K/V buffers are static LDS (128 KiB of the CU's 160 KiB).
     if (G == 1) hipLaunchKernelGGL(prefill_kernel<1>, grid, dim3(kNT), 0, st, a);
     else if (G == 2) hipLaunchKernelGGL(prefill_kernel<2>, grid, dim3(kNT), 0, st, a);

@@ -1,0 +1,73 @@
+"""GPU parity of the short-grid prefill launch (prefill_split_kernel: 16 or 32 query rows per
+workgroup, the keys shared out over its waves) against the oracle, at the edges of its query
+tiles (one query; a tile, a tile and one; the largest 16-row and the smallest and largest
+32-row grids of one sequence), with fewer batches of keys than waves, windows, block sizes and
+ragged counts; bad tables, inactive sequences and unwritten pool rows that are not finite.
+Same tolerance as the other prefill tests (2e-2, tests/parity.py)."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+from pkv import BF16, LayerSpec, hip, lib
+from pkv.engine import make_params
+from pkv.workloads import PrefillChunk
+from tests.test_gpu_prefill import _run
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("hq,hkv,prefix,counts,window", [
+    (16, 8, [0], [1], 0), (16, 8, [3], [8], 0), (16, 8, [120], [9], 0), (16, 8, [700], [17], 30),
+    (16, 8, [1000], [256], 0), (16, 8, [333], [257], 100), (16, 8, [50], [512], 0),
+    (16, 8, [0, 640], [1, 120], 0), (16, 8, [31, 250], [250, 33], 64), (8, 8, [77], [300], 0),
+    (8, 8, [900], [40], 128), (16, 4, [129], [100], 0), (16, 4, [260], [250], 90),
+    (16, 8, [16, 5, 900, 0], [7, 32, 1, 12], 0),
+])
+def test_prefill_split_matches_oracle(gpu, hq, hkv, prefix, counts, window):
+    print(f"[prefill split] {hq}q/{hkv}kv prefix={prefix} counts={counts} window={window}", flush=True)
+    w = PrefillChunk(seed=hq + sum(counts), batch=len(prefix), chunk=max(counts), prefix_max=max(prefix), hq=hq,
+                     hkv=hkv, window=window, prefix=prefix)
+    _run(w, q_counts=counts)
+
+
+@pytest.mark.parametrize("bs", [8, 32, 64])
+def test_prefill_split_block_sizes(gpu, bs):
+    print(f"[prefill split] block size {bs}", flush=True)
+
+    class Chunk(PrefillChunk):
+        BS = bs
+
+    _run(Chunk(seed=bs, batch=1, chunk=90, prefix_max=205, prefix=[205]))
+    _run(Chunk(seed=bs + 1, batch=1, chunk=300, prefix_max=13, prefix=[13]))
+
+
+@pytest.mark.parametrize("n", [12, 300], ids=["16-rows", "32-rows"])
+def test_prefill_split_contract_and_unwritten_rows(gpu, n):
+    print(f"[prefill split] contract, {n} queries", flush=True)
+    rng = np.random.default_rng(n)
+    hq, hkv, d, bs, nb, stride = 16, 8, 256, 16, 64, 40
+    p = make_params(LayerSpec(hq, hkv, d, kv_dtype=BF16), bs, nb, 0.0625)
+    q = hip.DeviceArray.from_numpy(O.to_bf16(rng.standard_normal((n, hq, d), dtype=np.float32)))
+    k = hip.DeviceArray((nb * bs, hkv * d), np.uint16, zero=True)
+    v = np.full((nb, bs, hkv * d), 0x7FC0, np.uint16)  # NaN in every row no key was written to
+    tables = rng.permutation(nb)[:stride].astype(np.int32).reshape(1, stride)
+    pos = 37
+    for t in range(pos + n):
+        v[tables[0, t // bs], t % bs] = 0x3F80  # 1.0
+    dv, out = hip.DeviceArray.from_numpy(v), hip.DeviceArray((n, hq, d), np.float32)
+    off = hip.DeviceArray.from_numpy(np.array([0, n], np.int32))
+
+    def call(tab, at, max_pos):
+        dt, dp = hip.DeviceArray.from_numpy(tab), hip.DeviceArray.from_numpy(np.array([at], np.int32))
+        lib.call("pkv_prefill", None, ctypes.byref(p), q.ptr, k.ptr, dv.ptr, dt.ptr, stride, dp.ptr, off.ptr, n, 1,
+                 max_pos, out.ptr)
+        return out.numpy()
+
+    assert np.allclose(call(tables, pos, 600), 1.0, atol=1e-6)  # equal weights of rows of ones
+    assert np.all(call(tables, -1, 600) == 0.0)                 # inactive
+    assert np.all(np.isnan(call(tables, pos, pos + n - 2)))     # past max_pos
+    bad = tables.copy()
+    bad[0, 1] = nb
+    assert np.all(np.isnan(call(bad, pos, 600)))                # an entry outside the pool
