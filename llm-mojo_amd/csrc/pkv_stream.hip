@@ -3021,7 +3021,159 @@ __global__ __launch_bounds__(merge_threads<D>()) void stream_merge_kernel(Stream
     }
 }
 
+// The same for few sequences cut into many pieces (one to a few sequences over the whole chip).
+// grid (rows_seq x D / kMergeDims, batch), plus one row of workgroups (blockIdx.y == batch)
+// with a fused append, whose first workgroup writes the state.
+// A workgroup combines 128 dims of one row: eight groups of 32 lanes take the pieces in turn,
+// four dims to a lane, and their sums meet in LDS. What bounds it is the round trips: after
+// the plan, the (m, l) and the o of the first 32 pieces are requested together, later pieces
+// 64 at a time, where one thread per dim walks them eight at a time: one sequence of 8000 keys
+// at head_dim 512 in 512 pieces 38.8 -> 14.2 us (fp32), 35.4 -> 11.8 us (bf16), four of 4000
+// keys in 128 pieces each 14.5 -> 8.2 us. With a few pieces per sequence the smaller
+// workgroups only repeat the plan and the weights (LSA's ~9 pieces: 7.2 -> 8.6 us).
+constexpr int kMergeNT = 256;
+constexpr int kMergeDims = 128;  // dims per workgroup
+template <int D, typename Acc>
+__global__ __launch_bounds__(kMergeNT) void stream_merge_many_kernel(StreamArgs a) {
+    constexpr int kMaxPieces = 1024;
+    constexpr int kSlices = D / kMergeDims;
+    constexpr int kGroups = kMergeNT / 32;  // piece groups of 32 lanes x 4 dims
+    constexpr int kRegs = 4;                // pieces per group requested with the (m, l)
+    constexpr int kTail = 8;                // pieces per group in flight after those
+    typedef Acc Acc4 __attribute__((ext_vector_type(4)));
+    __shared__ Acc s_w[kMaxPieces];
+    __shared__ Acc s_part[kMergeNT / kSW];
+    __shared__ Acc s_sum[kGroups][kMergeDims];
+    __shared__ int s_nan;
+    const int row = blockIdx.x / kSlices;
+    const int slice = blockIdx.x - row * kSlices;
+    const int s = blockIdx.y;
+    const int tid = threadIdx.x;
+    const int lane = tid & (kSW - 1);
+    const int wave = tid / kSW;
+    if (s == a.batch) {  // fused append
+        if (blockIdx.x == 0) write_alloc_state(a);
+        return;
+    }
+    if (row / a.Hq >= seq_queries(a, s)) return;  // a row past the sequence's queries
+    KeySplit sp;
+    sp.per_pair = a.plan[0];
+    sp.even = a.plan[1];
+    const int ps = a.plan[2 + s], pe = a.plan[3 + s];
+    if (pe == ps) return;
+    const int wf = sp.owner(ps + a.lead), wl = sp.owner(pe - 1);
+    if (wf == wl) return;
+    const int cnt = wl - wf + 1;  // <= nwg <= kMaxPieces
+    const Acc* pml = static_cast<const Acc*>(a.part_ml);
+    auto slot_row = [&](int c) -> size_t { return (size_t)(wf + c + s) * a.rows_seq + row; };
+    const int grp = tid / 32;                                    // takes pieces grp, grp + kGroups, ...
+    const int d4 = slice * kMergeDims + 4 * (tid & 31);          // this lane's first dim
+    const Acc* po = static_cast<const Acc*>(a.part_o) + d4;
+    auto o_of = [&](int c) -> Acc4 { return *reinterpret_cast<const Acc4*>(po + slot_row(c) * D); };
+
+    // Requests: (m, l) of this thread's pieces, o of the first pieces (a piece past the last
+    // re-reads the last one and takes no part).
+    Acc m0 = (Acc)-INFINITY, l0 = (Acc)0;
+    if (tid < cnt) {
+        m0 = pml[slot_row(tid) * 2];
+        l0 = pml[slot_row(tid) * 2 + 1];
+    }
+    Acc4 oreg[kRegs];
+#pragma unroll
+    for (int i = 0; i < kRegs; ++i) oreg[i] = o_of(min(grp + i * kGroups, cnt - 1));
+
+    if (tid == 0) s_nan = 0;
+    __syncthreads();
+    Acc M = (Acc)-INFINITY;
+    if (tid < cnt) {
+        if (m0 != m0) s_nan = 1;
+        M = m0;
+        s_w[tid] = m0;
+    }
+    for (int c = tid + kMergeNT; c < cnt; c += kMergeNT) {
+        const Acc m = pml[slot_row(c) * 2];
+        if (m != m) s_nan = 1;
+        M = fmax(M, m);
+        s_w[c] = m;
+    }
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) M = fmax(M, __shfl_xor(M, o));
+    if (lane == 0) s_part[wave] = M;
+    __syncthreads();
+    M = s_part[0];
+#pragma unroll
+    for (int i = 1; i < kMergeNT / kSW; ++i) M = fmax(M, s_part[i]);
+    __syncthreads();
+    Acc L = (Acc)0;
+    if (tid < cnt) {
+        const Acc wgt = (m0 == (Acc)-INFINITY) ? (Acc)0 : exp_acc(m0 - M);
+        s_w[tid] = wgt;
+        L = l0 * wgt;
+    }
+    for (int c = tid + kMergeNT; c < cnt; c += kMergeNT) {
+        const Acc m = s_w[c];
+        const Acc wgt = (m == (Acc)-INFINITY) ? (Acc)0 : exp_acc(m - M);
+        s_w[c] = wgt;
+        L += pml[slot_row(c) * 2 + 1] * wgt;
+    }
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) L += __shfl_xor(L, o);
+    if (lane == 0) s_part[wave] = L;
+    __syncthreads();
+    L = (Acc)0;
+#pragma unroll
+    for (int i = 0; i < kMergeNT / kSW; ++i) L += s_part[i];
+    Acc4 sum = {(Acc)0, (Acc)0, (Acc)0, (Acc)0};
+#pragma unroll
+    for (int i = 0; i < kRegs; ++i) {
+        const int c = grp + i * kGroups;
+        if (c < cnt) {
+            const Acc wgt = s_w[c];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) sum[e] = fma(wgt, oreg[i][e], sum[e]);
+        }
+    }
+    for (int c0 = kRegs * kGroups; c0 < cnt; c0 += kTail * kGroups) {
+        Acc4 x[kTail];
+#pragma unroll
+        for (int i = 0; i < kTail; ++i) x[i] = o_of(min(c0 + grp + i * kGroups, cnt - 1));
+#pragma unroll
+        for (int i = 0; i < kTail; ++i) {
+            const int c = c0 + grp + i * kGroups;
+            if (c < cnt) {
+                const Acc wgt = s_w[c];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) sum[e] = fma(wgt, x[i][e], sum[e]);
+            }
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) s_sum[grp][4 * (tid & 31) + e] = sum[e];
+    __syncthreads();
+    if (tid < kMergeDims) {
+        Acc o = (Acc)0;
+#pragma unroll
+        for (int i = 0; i < kGroups; ++i) o += s_sum[i][tid];
+        const Acc inv = (Acc)1 / (L + (Acc)1e-10);
+        a.out[(((size_t)s * a.q_len + a.j0) * a.Hq + row) * D + slice * kMergeDims + tid] =
+            s_nan != 0 ? __builtin_nanf("") : (float)(o * inv);
+    }
+}
+
 // ---- host -------------------------------------------------------------------------
+
+// The merge of a launch of a.nwg workgroups along the keys. A sequence has about
+// a.nwg / batch pieces; from 32 on they are combined by stream_merge_many_kernel (128 pieces
+// 14.5 -> 8.2 us; at 16 the two take the same, 10.6 and 10.3 us).
+template <int D, typename Acc>
+void launch_merge(const StreamArgs& a, bool fused, hipStream_t st) {
+    const int rows = a.batch + (fused ? 1 : 0);
+    if (a.nwg >= 32 * (int64_t)a.batch)
+        hipLaunchKernelGGL((stream_merge_many_kernel<D, Acc>), dim3(a.rows_seq * (D / kMergeDims), rows), dim3(kMergeNT),
+                           0, st, a);
+    else
+        hipLaunchKernelGGL((stream_merge_kernel<D, Acc>), dim3(a.rows_seq, rows), dim3(merge_threads<D>()), 0, st, a);
+}
 
 constexpr int kMaxSlots = kStreamMaxSlots;  // workgroups along the keys, at most (merge LDS bound)
 
@@ -3060,8 +3212,7 @@ int32_t launch_addr(StreamArgs a, hipStream_t st) {
                                dim3(kMaxWaves * kSW), lds_iw, st, a);
             if (hipGetLastError() != hipSuccess)
                 return fail(PKV_ERR_HIP, "pkv_attend: the attention launch failed");
-            hipLaunchKernelGGL((stream_merge_kernel<D, Acc>), dim3(a.rows_seq, a.batch + (fused ? 1 : 0)),
-                               dim3(merge_threads<D>()), 0, st, a);
+            launch_merge<D, Acc>(a, fused, st);
             return PKV_OK;
         }
     }
@@ -3087,8 +3238,7 @@ int32_t launch_addr(StreamArgs a, hipStream_t st) {
     // the merge reads the plan this launch writes
     if (hipGetLastError() != hipSuccess)
         return fail(PKV_ERR_HIP, "pkv_attend: the attention launch failed");
-    hipLaunchKernelGGL((stream_merge_kernel<D, Acc>), dim3(a.rows_seq, a.batch + (fused ? 1 : 0)),
-                       dim3(merge_threads<D>()), 0, st, a);
+    launch_merge<D, Acc>(a, fused, st);
     return PKV_OK;
 }
 
@@ -3135,8 +3285,7 @@ bool launch_mfma_iw(StreamArgs& a, hipStream_t st, int32_t* rc) {
         *rc = fail(PKV_ERR_HIP, "pkv_attend: the attention launch failed");
         return true;
     }
-    hipLaunchKernelGGL((stream_merge_kernel<D, double>), dim3(a.rows_seq, a.batch + (fused ? 1 : 0)),
-                       dim3(merge_threads<D>()), 0, st, a);
+    launch_merge<D, double>(a, fused, st);
     *rc = PKV_OK;
     return true;
 }
@@ -3178,8 +3327,7 @@ int32_t launch_mfma_addr(StreamArgs a, hipStream_t st) {
         hipLaunchKernelGGL((stream_mfma_kernel<D, RG, TG, WPH, ADDR, false>), grid, dim3(threads), lds, st, a);
     if (hipGetLastError() != hipSuccess)
         return fail(PKV_ERR_HIP, "pkv_attend: the attention launch failed");
-    hipLaunchKernelGGL((stream_merge_kernel<D, double>), dim3(a.rows_seq, a.batch + (fused ? 1 : 0)),
-                       dim3(merge_threads<D>()), 0, st, a);
+    launch_merge<D, double>(a, fused, st);
     return PKV_OK;
 }
 
@@ -3224,8 +3372,7 @@ int32_t launch_bf16_mfma(StreamArgs a, hipStream_t st) {
                            lds_iw, st, a);
         if (hipGetLastError() != hipSuccess)
             return fail(PKV_ERR_HIP, "pkv_attend: the attention launch failed");
-        hipLaunchKernelGGL((stream_merge_kernel<256, float>), dim3(a.rows_seq, a.batch), dim3(merge_threads<256>()), 0,
-                           st, a);
+        launch_merge<256, float>(a, false, st);
         return PKV_OK;
     }
     const void* fn = reinterpret_cast<const void*>(&stream_bf16_mfma_kernel<kAddrPaged>);
@@ -3242,8 +3389,7 @@ int32_t launch_bf16_mfma(StreamArgs a, hipStream_t st) {
                        st, a);
     if (hipGetLastError() != hipSuccess)
         return fail(PKV_ERR_HIP, "pkv_attend: the attention launch failed");
-    hipLaunchKernelGGL((stream_merge_kernel<256, float>), dim3(a.rows_seq, a.batch), dim3(merge_threads<256>()), 0,
-                       st, a);
+    launch_merge<256, float>(a, false, st);
     return PKV_OK;
 }
 
@@ -3269,8 +3415,7 @@ int32_t launch_rows_kernel(StreamArgs a, hipStream_t st) {
     hipLaunchKernelGGL((stream_rows_kernel<D, RT, ADDR>), dim3(a.nwg, a.Hkv), dim3(kMaxWaves * kSW), lds, st, a);
     if (hipGetLastError() != hipSuccess)
         return fail(PKV_ERR_HIP, "pkv_attend: the attention launch failed");
-    hipLaunchKernelGGL((stream_merge_kernel<D, double>), dim3(a.rows_seq, a.batch), dim3(merge_threads<D>()), 0, st,
-                       a);
+    launch_merge<D, double>(a, false, st);
     return PKV_OK;
 }
 template <int D, int RT>
