@@ -299,7 +299,7 @@ size_t pkv_lsa_expand_workspace_size(int32_t batch, int32_t top_k, int32_t sink_
  * int32 [batch + 1]. keys_capacity (int32 entries) must be >= batch *
  * pkv_lsa_max_keys(). status[s] = PKV_SEQ_BAD_INDEX when the index id, n_picked or a
  * bucket id is out of range (the offending part is skipped), else PKV_SEQ_OK. All arrays
- * are device memory; batch <= 1024; sink_size, window_size >= 0. Two launches. */
+ * are device memory; batch <= 1024; sink_size, window_size >= 0. One or two launches. */
 int32_t pkv_lsa_expand(void* stream, const int32_t* index_ids, const int32_t* picked,
                        int32_t picked_stride, const int32_t* n_picked, const int32_t* pos,
                        int32_t top_k, int32_t sink_size, int32_t window_size, int32_t batch,

@@ -10,13 +10,19 @@
 // closed_blocks[i] and total_tokens[i]. Building buckets when a 512-token block closes
 // (Ward clustering) and picking them (select_top_p) stay with the index on the host.
 //
-// pkv_lsa_expand is two launches. lsa_gather_kernel gives each sequence one wave: the
-// picked ids and sizes of up to 64 buckets come in one load per lane, then every member row
-// of those buckets in one round trip into LDS, and the filter walks them in order (one
-// ballot per bucket keeps the members' order) into a fixed-stride staging area of the
-// workspace. lsa_compact_kernel, one workgroup, scans the lengths into key_off and copies
-// the lists end to end (CSR). lsa_rollback_kernel: one workgroup applying the entries in
-// order, so repeated index ids behave like repeated calls.
+// pkv_lsa_expand. One wave builds a sequence's list: its ids, pick count and picks come in one
+// round trip, the sizes and member rows of up to 32 picked buckets in the next (a bucket to a
+// half-wave, straight into registers), and one ballot per two buckets keeps the members' order.
+//   Up to kLsaOneBatch sequences whose lists fit in LDS: one workgroup, one launch. The lists
+//     stay in LDS, a scan of their lengths gives key_off, and they go out end to end.
+//   Else two launches: lsa_gather_kernel, one wave per sequence, into a fixed-stride staging
+//     area of the workspace; lsa_compact_kernel, one workgroup per sequence, adds up the lengths
+//     before its own and copies its list (CSR).
+// What bounds both is latency. Against members staged in LDS after four dependent round trips
+// and one workgroup compacting: 1 sequence of 20 buckets 11.6 -> 5.8 us, 5 14.3 -> 6.8 us (one
+// launch), 33 18.6 -> 9.7 us, 64 21.4 -> 10.8 us (two).
+// lsa_rollback_kernel: one workgroup applying the entries in order, so repeated index ids behave
+// like repeated calls.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -28,10 +34,14 @@ namespace {
 constexpr int kLsaBucketCap = 32;       // LSA_BUCKET_CAP (lsa_core.mojo:27)
 constexpr int kLsaBlockBuckets = 32;    // LSA_BLOCK_BUCKET_COUNT (lsa_core.mojo:28)
 constexpr int kLsaClusterBlock = 512;   // LSA_CLUSTER_BLOCK_SIZE (lsa_core.mojo:26)
-constexpr int kLsaCompactThreads = 1024;
-constexpr int kLsaCompactWaves = kLsaCompactThreads / 64;
-constexpr int kLsaMaxBatch = kLsaCompactThreads;  // one scan element per thread
-constexpr int kLsaChunk = 64;                     // picked buckets staged per round
+constexpr int kLsaMaxBatch = 1024;
+constexpr int kLsaChunk = 32;           // picked buckets per round (two to a load)
+// The one-launch form: a wave per sequence (16 sequences, two to a wave, took the same 9.6 us
+// as two launches, 32 took 16.6 against 9.7).
+constexpr int kLsaOneBatch = 8;
+constexpr int kLsaOneThreads = 64 * kLsaOneBatch;
+constexpr size_t kLsaOneLds = 60 * 1024;  // of lists
+constexpr int kLsaCompactThreads = 256;
 
 struct LsaExpandArgs {
     const int32_t* index_ids;  // [batch]
@@ -55,19 +65,21 @@ struct LsaExpandArgs {
     int32_t max_buckets;
 };
 
-// One wave per sequence s = blockIdx.x.
-__global__ __launch_bounds__(64) void lsa_gather_kernel(LsaExpandArgs a) {
-    __shared__ int s_b[kLsaChunk], s_size[kLsaChunk];
-    __shared__ int s_tok[kLsaChunk][kLsaBucketCap];
-    const int s = blockIdx.x, lane = threadIdx.x;
-    int32_t* out = a.stage + (size_t)s * a.per;
+// Sequence s's list into out (one wave; out in LDS or global memory). Returns its length and
+// writes the sequence's status.
+__device__ inline int lsa_build_list(const LsaExpandArgs& a, int s, int lane, int32_t* out) {
+    const int half = lane >> 5, m32 = lane & (kLsaBucketCap - 1);
+    const int pick_last = a.picked_stride - 1;
+    // one round trip: every load is issued, indices clamped into range
     const int p = a.pos[s];
-    const int ws = max(0, p + 1 - a.window);  // window start (lsa_core.mojo:577)
     const int idx = a.index_ids[s];
+    const int np_raw = a.n_picked[s];
+    int pick = pick_last >= 0 ? a.picked[(size_t)s * a.picked_stride + min(lane, pick_last)] : -1;
+    const int ws = max(0, p + 1 - a.window);  // window start (lsa_core.mojo:577)
     bool bad = false;
     int n = 0;
     if (idx >= 0 && idx < a.num_indices) {
-        int np = a.n_picked[s];
+        int np = np_raw;
         if (np < 0 || np > a.picked_stride) {
             bad = true;
             np = max(0, min(np, a.picked_stride));
@@ -80,40 +92,40 @@ __global__ __launch_bounds__(64) void lsa_gather_kernel(LsaExpandArgs a) {
         bool stop = false;
         for (int j0 = 0; j0 < np && !stop; j0 += kLsaChunk) {
             const int cnt = min(kLsaChunk, np - j0);
-            int b = -1, size = 0;
-            if (lane < cnt) b = a.picked[(size_t)s * a.picked_stride + j0 + lane];
-            if (lane < cnt && b >= 0 && b < a.max_buckets) size = min(max(sz[b], 0), kLsaBucketCap);
-            s_b[lane] = b;
-            s_size[lane] = size;
-            __syncthreads();
-            for (int t = lane; t < cnt * kLsaBucketCap; t += 64) {
-                const int j = t / kLsaBucketCap, m = t % kLsaBucketCap;
-                s_tok[j][m] = m < s_size[j] ? mem[(size_t)s_b[j] * kLsaBucketCap + m] : 0;
-            }
-            __syncthreads();
-            for (int j = 0; j < cnt; ++j) {
-                if (j0 + j > 0 && n >= a.top_k) {
-                    stop = true;
-                    break;
-                }
-                const int bj = s_b[j];
-                if (bj < 0 || bj >= a.max_buckets) {
-                    bad = true;
-                    continue;
-                }
-                int tok = 0;
-                bool keep = false;
-                if (lane < s_size[j]) {
-                    tok = s_tok[j][lane];
-                    keep = tok >= a.sink && tok < ws;
-                }
+            if (j0 > 0) pick = a.picked[(size_t)s * a.picked_stride + min(j0 + lane, pick_last)];
+            const bool pick_ok = lane < cnt && pick >= 0 && pick < a.max_buckets;
+            const int b = pick_ok ? pick : 0;
+            const int size_raw = sz[b];
+            int tok[kLsaChunk / 2];  // bucket 2i + half, member m32
+#pragma unroll
+            for (int i = 0; i < kLsaChunk / 2; ++i)
+                if (2 * i < cnt) tok[i] = mem[(size_t)__shfl(b, 2 * i + half) * kLsaBucketCap + m32];
+            const int size = pick_ok ? min(max(size_raw, 0), kLsaBucketCap) : 0;
+            const uint64_t valid = __ballot(pick_ok);
+#pragma unroll
+            for (int i = 0; i < kLsaChunk / 2; ++i) {
+                if (2 * i >= cnt || stop) break;
+                const bool keep = m32 < __shfl(size, 2 * i + half) && tok[i] >= a.sink && tok[i] < ws;
                 const uint64_t mask = __ballot(keep);
-                const int rank = __popcll(mask & ((1ull << lane) - 1ull));
-                const int take = min(__popcll(mask), max(a.top_k - n, 1));
-                if (keep && rank < take) out[n + rank] = tok;
-                n += take;
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const int j = 2 * i + h;
+                    if (j >= cnt || stop) break;
+                    if (j0 + j > 0 && n >= a.top_k) {
+                        stop = true;
+                        break;
+                    }
+                    if (!((valid >> j) & 1)) {
+                        bad = true;
+                        continue;
+                    }
+                    const uint32_t mine = (uint32_t)(mask >> (32 * h));
+                    const int take = min(__popc(mine), max(a.top_k - n, 1));
+                    const int rank = __popc(mine & ((1u << m32) - 1u));
+                    if (half == h && keep && rank < take) out[n + rank] = tok[i];
+                    n += take;
+                }
             }
-            __syncthreads();  // the next chunk overwrites the staged rows
         }
     } else {
         bad = true;
@@ -125,43 +137,55 @@ __global__ __launch_bounds__(64) void lsa_gather_kernel(LsaExpandArgs a) {
     // 3. the sinks [0, min(sink, ws, p + 1))
     const int scnt = max(0, min(min(a.sink, ws), p + 1));
     for (int t = lane; t < scnt; t += 64) out[n + t] = t;
+    if (lane == 0) a.status[s] = bad ? PKV_SEQ_BAD_INDEX : PKV_SEQ_OK;
+    return n + scnt;
+}
+
+// The whole call in one workgroup: lists in LDS ([batch][per]), then their offsets.
+__global__ __launch_bounds__(kLsaOneThreads) void lsa_expand_kernel(LsaExpandArgs a) {
+    extern __shared__ int32_t s_list[];
+    __shared__ int s_len[kLsaOneBatch];
+    const int lane = threadIdx.x & 63, s = threadIdx.x >> 6;
+    int n = 0;
+    if (s < a.batch) n = lsa_build_list(a, s, lane, s_list + (size_t)s * a.per);
+    if (lane == 0) s_len[s] = n;
+    __syncthreads();
+    if (s >= a.batch) return;
+    int base = 0;
+    for (int i = 0; i < s; ++i) base += s_len[i];
+    for (int t = lane; t < n; t += 64) a.keys[base + t] = s_list[(size_t)s * a.per + t];
     if (lane == 0) {
-        a.len[s] = n + scnt;
-        a.status[s] = bad ? PKV_SEQ_BAD_INDEX : PKV_SEQ_OK;
+        a.key_off[s] = base;
+        if (s == a.batch - 1) a.key_off[a.batch] = base + n;
     }
 }
 
-// Scan of the lengths into key_off, then the lists end to end into keys.
+// One wave per sequence s = blockIdx.x.
+__global__ __launch_bounds__(64) void lsa_gather_kernel(LsaExpandArgs a) {
+    const int s = blockIdx.x, lane = threadIdx.x;
+    const int n = lsa_build_list(a, s, lane, a.stage + (size_t)s * a.per);
+    if (lane == 0) a.len[s] = n;
+}
+
+// Sequence s = blockIdx.x: its offset (the lengths before it), then its list into keys.
 __global__ __launch_bounds__(kLsaCompactThreads) void lsa_compact_kernel(LsaExpandArgs a) {
-    __shared__ int s_off[kLsaMaxBatch];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    s_off[tid] = tid < a.batch ? a.len[tid] : 0;
+    __shared__ int s_part[kLsaCompactThreads / 64];
+    const int s = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int n = a.len[s];
+    int base = 0;
+    for (int i = tid; i < s; i += kLsaCompactThreads) base += a.len[i];
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) base += __shfl_xor(base, o);
+    if (lane == 0) s_part[wave] = base;
     __syncthreads();
-    for (int d = 1; d < kLsaMaxBatch; d <<= 1) {  // inclusive Hillis-Steele scan
-        const int t = tid >= d ? s_off[tid - d] : 0;
-        __syncthreads();
-        s_off[tid] += t;
-        __syncthreads();
-    }
-    if (tid < a.batch) a.key_off[tid + 1] = s_off[tid];
-    if (tid == 0) a.key_off[0] = 0;
-    for (int s = wave; s < a.batch; s += kLsaCompactWaves) {
-        const int base = s == 0 ? 0 : s_off[s - 1];
-        const int n = s_off[s] - base;
-        const int32_t* src = a.stage + (size_t)s * a.per;
-        for (int t0 = 0; t0 < n; t0 += 4 * 64) {  // four loads in flight per lane
-            int v[4];
+    base = 0;
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int t = t0 + u * 64 + lane;
-                v[u] = t < n ? src[t] : 0;
-            }
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int t = t0 + u * 64 + lane;
-                if (t < n) a.keys[base + t] = v[u];
-            }
-        }
+    for (int i = 0; i < kLsaCompactThreads / 64; ++i) base += s_part[i];
+    const int32_t* src = a.stage + (size_t)s * a.per;
+    for (int t = tid; t < n; t += kLsaCompactThreads) a.keys[base + t] = src[t];
+    if (tid == 0) {
+        a.key_off[s] = base;
+        if (s == a.batch - 1) a.key_off[a.batch] = base + n;
     }
 }
 
@@ -270,8 +294,13 @@ int32_t pkv_lsa_expand(void* stream, const int32_t* index_ids, const int32_t* pi
     a.num_indices = num_indices;
     a.max_buckets = max_buckets;
     hipStream_t st = static_cast<hipStream_t>(stream);
+    const size_t lists = (size_t)batch * per * sizeof(int32_t);
+    if (batch <= kLsaOneBatch && lists <= kLsaOneLds) {
+        hipLaunchKernelGGL(lsa_expand_kernel, dim3(1), dim3(kLsaOneThreads), lists, st, a);
+        return check_launch("pkv_lsa_expand");
+    }
     hipLaunchKernelGGL(lsa_gather_kernel, dim3(batch), dim3(64), 0, st, a);
-    hipLaunchKernelGGL(lsa_compact_kernel, dim3(1), dim3(kLsaCompactThreads), 0, st, a);
+    hipLaunchKernelGGL(lsa_compact_kernel, dim3(batch), dim3(kLsaCompactThreads), 0, st, a);
     return check_launch("pkv_lsa_expand");
 }
 

@@ -97,6 +97,28 @@ def test_expand_matches_oracle(gpu, top_k, sink, window):
     np.testing.assert_array_equal(got_status, want_status)
 
 
+@pytest.mark.parametrize("batch,stride,top_k", [(1, 20, 256), (8, 33, 700), (8, 3, 1), (9, 20, 256), (65, 31, 90),
+                                                (5, 70, 900)])
+def test_expand_one_and_two_launches(gpu, batch, stride, top_k):
+    # Up to 8 sequences take one launch, more two; picks past a round of 32 buckets, odd and
+    # empty pick lists, lists cut inside the first and the second bucket of a pair.
+    print(f"[lsa-cache] expand batch={batch} stride={stride} top_k={top_k}", flush=True)
+    rng = np.random.default_rng(batch * 100 + stride)
+    nidx, max_capacity, sink, window = 6, 4096, 4, 128
+    cache = LSABucketCache(nidx, max_capacity)
+    sizes, members = _fill(rng, nidx, max_capacity, 3000)
+    _upload(cache, sizes, members)
+    ids = rng.integers(0, nidx, batch)
+    n_picked = rng.integers(0, stride + 1, batch)
+    n_picked[0] = stride
+    picked = rng.integers(0, cache.max_buckets, (batch, stride))
+    pos = rng.integers(0, 3000, batch)
+    got = _expand(cache, ids, picked, n_picked, pos, top_k, sink, window)
+    want = _expected(sizes, members, ids, picked, n_picked, pos, top_k, sink, window, nidx, cache.max_buckets)
+    for g, w in zip(got, want):
+        np.testing.assert_array_equal(g, w)
+
+
 def test_expand_flags_bad_ids(gpu):
     print("[lsa-cache] bad index / bucket ids, n_picked past the stride", flush=True)
     rng = np.random.default_rng(11)
