@@ -459,6 +459,126 @@ void q4_matmul_kernel(Q4Args a) {
     }
 }
 
+// A few sequences (decode of one or two chats): the split x fits in LDS, so a workgroup takes 16
+// rows over all of K and nothing is left to add up between workgroups. Its sixteen waves take
+// the rows' blocks in runs: a wave's weights are requested first, the
+// workgroup splits x into its three exact bf16 parts once meanwhile, then every block is three
+// MFMAs on operands from LDS, scaled and summed as in q4_matmul_kernel. The waves' sums are added in wave order.
+// One sequence, back to back: 4096 -> 2816 11.9 -> 6.7 us, 8192 -> 2816 12.9 -> 9.4 us. What
+// bounds it is the chain launch, x (L2), split, blocks, sum: the weights alone take 1-2 us of
+// HBM. (Weights a dword per lane, 16 bytes of a row at a time: 19.6 us, all in the address path.)
+constexpr int kQ4sWaves = 16;
+constexpr int kQ4sNT = kQ4sWaves * 64;
+constexpr int kQ4sMaxBatch = 4;            // one quad of sequences: the lanes of quarter 0 hold the sums
+constexpr size_t kQ4sLds = 128 * 1024;     // of split x
+constexpr int kQ4sRun = 8;                 // blocks per round of a wave, two rounds requested ahead
+__host__ __device__ inline size_t q4s_row_bytes(int c_in) { return (size_t)c_in * 2 + 64; }  // one part of one sequence
+__host__ __device__ inline size_t q4s_x_bytes(int c_in, int batch) { return 3 * (size_t)batch * q4s_row_bytes(c_in); }
+// then the rows' scales, [16][nb + 1]
+__host__ __device__ inline size_t q4s_lds(int c_in, int batch) {
+    return q4s_x_bytes(c_in, batch) + 16 * ((size_t)c_in / 32 + 1) * sizeof(float);
+}
+
+__global__ __launch_bounds__(kQ4sNT) void q4_small_kernel(Q4Args a) {
+    extern __shared__ __attribute__((aligned(16))) char s_x[];  // [part][sequence][c_in] bf16
+    __shared__ float s_sum[kQ4sWaves][kQ4sMaxBatch][16];
+    const int tid = threadIdx.x, lane = tid & 63, v = tid >> 6;
+    const int j = lane & 15, q = lane >> 4;
+    const int row = min((int)blockIdx.x * 16 + j, a.c_out - 1);
+    const int per = (a.nb + kQ4sWaves - 1) / kQ4sWaves;
+    const int b_lo = v * per, b_hi = min(a.nb, b_lo + per);
+    const uint4* wr = reinterpret_cast<const uint4*>(a.w + (size_t)row * (a.c_in / 2));
+    float* const s_sc = reinterpret_cast<float*>(s_x + q4s_x_bytes(a.c_in, a.batch));
+
+    // Lane (j, q) loads blocks b0 + 4i + q of row j whole (16 rows x 64 contiguous bytes a load);
+    // a 4 x 4 transpose over the lane quarters then leaves dword q of block b0 + i in w[i].
+    // Blocks past the row re-read its last one and are not used.
+    uint4 wn[2][kQ4sRun / 4];  // the next two rounds
+    auto load = [&](uint4 (&d)[kQ4sRun / 4], int b0) {
+#pragma unroll
+        for (int i = 0; i < kQ4sRun / 4; ++i) d[i] = wr[min(b0 + 4 * i + q, a.nb - 1)];
+    };
+    uint32_t w[kQ4sRun];
+    auto transpose = [&](const uint4 (&d)[kQ4sRun / 4]) {
+#pragma unroll
+        for (int i = 0; i < kQ4sRun; i += 4) {
+            w[i] = d[i / 4].x, w[i + 1] = d[i / 4].y, w[i + 2] = d[i / 4].z, w[i + 3] = d[i / 4].w;
+            auto p = __builtin_amdgcn_permlane32_swap(w[i], w[i + 2], false, false);
+            w[i] = p[0], w[i + 2] = p[1];
+            p = __builtin_amdgcn_permlane32_swap(w[i + 1], w[i + 3], false, false);
+            w[i + 1] = p[0], w[i + 3] = p[1];
+            p = __builtin_amdgcn_permlane16_swap(w[i], w[i + 1], false, false);
+            w[i] = p[0], w[i + 1] = p[1];
+            p = __builtin_amdgcn_permlane16_swap(w[i + 2], w[i + 3], false, false);
+            w[i + 2] = p[0], w[i + 3] = p[1];
+        }
+    };
+    load(wn[0], b_lo);
+    load(wn[1], b_lo + kQ4sRun);
+    for (int r = v; r < 16; r += kQ4sWaves) {  // the rows' scales, a row to a wave
+        const float* sr = a.scales + (size_t)min((int)blockIdx.x * 16 + r, a.c_out - 1) * a.nb;
+        for (int b = lane; b < a.nb; b += 64) s_sc[r * (a.nb + 1) + b] = sr[b];
+    }
+    const int units = a.c_in / 8;
+    const size_t rb = q4s_row_bytes(a.c_in);
+    for (int u = tid; u < units * a.batch; u += kQ4sNT) {
+        const int seq = u / units, e = u - seq * units;
+        const f32x4* xp = reinterpret_cast<const f32x4*>(a.x + (size_t)seq * a.c_in + 8 * e);
+        const f32x4 x0 = xp[0], x1 = xp[1];
+        const float xv[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+        bf16x8 h, m, l;
+        split3(xv, h, m, l);
+        char* d = s_x + (size_t)seq * rb + 16 * e;
+        *reinterpret_cast<bf16x8*>(d) = h;
+        *reinterpret_cast<bf16x8*>(d + a.batch * rb) = m;
+        *reinterpret_cast<bf16x8*>(d + 2 * a.batch * rb) = l;
+    }
+    __syncthreads();
+
+    f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+    const char* xq = s_x + (size_t)min(j, a.batch - 1) * rb + 16 * q;  // sequence j's inputs 8q .. of block 0
+    for (int b0 = b_lo; b0 < b_hi; b0 += kQ4sRun) {
+        transpose(wn[0]);
+#pragma unroll
+        for (int i = 0; i < kQ4sRun / 4; ++i) wn[0][i] = wn[1][i];
+        if (b0 + 2 * kQ4sRun < b_hi) load(wn[1], b0 + 2 * kQ4sRun);
+        const int n = b_hi - b0;
+#pragma unroll
+        for (int i = 0; i < kQ4sRun; ++i) {
+            // (a block past the run is not added)
+            const float sc = s_sc[j * (a.nb + 1) + min(b0 + i, a.nb - 1)] * kQ4Unpack;
+            const char* xb = xq + 64 * (size_t)min(b0 + i, a.nb - 1);
+            const bf16x8 h = *reinterpret_cast<const bf16x8*>(xb);
+            const bf16x8 m = *reinterpret_cast<const bf16x8*>(xb + a.batch * rb);
+            const bf16x8 l = *reinterpret_cast<const bf16x8*>(xb + 2 * a.batch * rb);
+            const bf16x8 W = unpack_q4(w[i]);
+            f32x4 c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(l, W, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+            c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(m, W, c, 0, 0, 0);
+            c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(h, W, c, 0, 0, 0);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float sum = fmaf(sc, c[e], acc[e]);
+                acc[e] = i < n ? sum : acc[e];
+            }
+        }
+        // keep the last sums in the MFMAs' basic block (see q4_matmul_kernel)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) asm volatile("" : "+v"(acc[e]));
+    }
+    if (q == 0) {
+#pragma unroll
+        for (int e = 0; e < kQ4sMaxBatch; ++e) s_sum[v][e][j] = acc[e];
+    }
+    __syncthreads();
+    if (tid < 16 * a.batch) {
+        const int seq = tid >> 4, r = blockIdx.x * 16 + j;
+        float sum = s_sum[0][seq][j];
+#pragma unroll
+        for (int x = 1; x < kQ4sWaves; ++x) sum += s_sum[x][seq][j];
+        if (r < a.c_out) a.out[(size_t)seq * a.c_out + r] = sum;
+    }
+}
+
 // Rows of a group in halves of 64: one. 64-row groups need at most 128 VGPRs up to two
 // column tiles, so two 8-wave workgroups share a CU (four waves per SIMD); 128-row groups
 // (two halves) measured slower at one workgroup per CU.
@@ -525,6 +645,23 @@ int32_t pkv_q4_matmul(void* stream, const uint8_t* w_packed, const float* scales
     a.arrived = static_cast<int32_t*>(workspace);
     a.part = reinterpret_cast<float*>(static_cast<char*>(workspace) +
                                       (((size_t)a.groups * sizeof(int32_t) + 255) & ~(size_t)255));
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    // A few sequences whose split x fits in LDS: 16 rows over all of K per workgroup, as long
+    // as those workgroups all run at once (one sequence, 4096 inputs: 2816 rows 11.9 -> 6.7 us,
+    // 16384 rows, two rounds, 18.5 against 19.0 us; 65536 rows of four sequences 52 against 101).
+    if (batch <= kQ4sMaxBatch && q4s_lds(c_in, batch) <= kQ4sLds) {
+        const size_t lds = q4s_lds(c_in, batch);
+        const void* small = reinterpret_cast<const void*>(&q4_small_kernel);
+        if (lds > 60 * 1024 && !reserve_lds(small, (int)kQ4sLds))
+            return fail(PKV_ERR_HIP, "pkv_q4_matmul: could not reserve the kernel's LDS");
+        const int resident = device_fill_workgroups(small, kQ4sNT, lds, INT32_MAX);
+        if (resident <= 0) return fail(PKV_ERR_HIP, "pkv_q4_matmul: occupancy query failed");
+        const int wgs = (c_out - 1) / 16 + 1;
+        if (wgs <= resident) {
+            hipLaunchKernelGGL(q4_small_kernel, dim3(wgs), dim3(kQ4sNT), lds, st, a);
+            return check_launch("pkv_q4_matmul");
+        }
+    }
     const int fill = device_fill_workgroups(fn, kQ4NT, 0, kQ4MaxWg);
     if (fill <= 0) return fail(PKV_ERR_HIP, "pkv_q4_matmul: occupancy query failed");
     // Splits per row group: as many as keep every workgroup resident in one round.
@@ -533,7 +670,6 @@ int32_t pkv_q4_matmul(void* stream, const uint8_t* w_packed, const float* scales
     if (splits > a.nb) splits = a.nb;
     a.per = (a.nb + splits - 1) / splits;
     a.splits = (a.nb + a.per - 1) / a.per;
-    hipStream_t st = static_cast<hipStream_t>(stream);
     // passes of 8 blocks per chunk: a run of `per` blocks in chunks of up to kQ4MaxPass
     const int passes = a.per >= 8 * kQ4MaxPass ? kQ4MaxPass : (a.per + 7) / 8;
     const dim3 grid(a.groups * a.splits), block(kQ4NT);
