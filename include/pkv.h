@@ -242,7 +242,7 @@ int32_t pkv_attend_noalloc(void* stream, const pkv_params* p, const float* q,
  * q_lens[s] - 1. Workspace: pkv_workspace_size(p, batch, max_q_len, max_pos). head_dim
  * 256 or 512 with num_heads / num_kv_heads <= 8 (every geometry of the engine); other
  * geometries give PKV_ERR_UNSUPPORTED. Two launches per group of up to 8 query rows per
- * kv head (fp32 pools: up to 32). */
+ * kv head (fp32 pools: up to 32; paged bf16 pools at head_dim 256: up to 16). */
 int32_t pkv_verify(void* stream, const pkv_params* p, const float* q, const void* k_pool,
                    const void* v_pool, const int32_t* block_tables, int32_t table_stride,
                    const int32_t* pos, const int32_t* q_lens, int32_t max_q_len, int32_t batch,

@@ -2348,7 +2348,7 @@ __global__ __launch_bounds__(kMaxWaves * kSW, 2) void stream_rows_kernel(StreamA
     }
 }
 
-// ---- bf16 MFMA path: bf16 pools, head_dim 256, 5..8 query rows per KV head -------------
+// ---- bf16 MFMA path: bf16 pools, head_dim 256, 5..16 query rows per KV head ------------
 //
 // One wave per KV head, up to 8 query rows (a 4-token verify at G = 2), batches of 16
 // tokens staged in LDS, all products on v_mfma_f32_16x16x32_bf16 (QK^T) and
@@ -2370,6 +2370,13 @@ __global__ __launch_bounds__(kMaxWaves * kSW, 2) void stream_rows_kernel(StreamA
 //     4 (a % 4) .. + 3 of token 4 (L / 16) + a / 4; inside each 16-lane group output lane j
 //     element e is element j % 4 of what input lane 4e + j / 4 addressed). The hi and lo
 //     columns are added once, at the end.
+// Nine to 16 rows (WIDE) fill the 16 columns with rows, and Q and P enter as three bf16 parts
+// of 8 significant bits (exact: the sums alone round), one instruction each into the same
+// accumulator, so O^T takes the same registers and nothing is folded. The keys' bytes bound it
+// (5.3 TB/s in the trace), so one pass instead of two halves the time of the second group, and
+// the third part costs nothing: 16 sequences of 512..4096 keys, 1..5 tokens at G = 2,
+// 60.5 + 4.7 (8 rows) + 20.6 + 5.3 us (2 rows) -> 62 + 5.0 us; error against
+// 64 bits 5.0e-6 -> 5.0e-7.
 // LDS per wave: K and V of 16 tokens, rows of 512 bytes; K's 16-byte chunk c of token r
 // sits at c ^ r and V's 32-byte chunk c at c ^ r, so the operand reads land on distinct
 // banks. A copy instruction moves two tokens (1 KiB): the batches start on even positions
@@ -2395,6 +2402,19 @@ __device__ inline uint16_t bf16_rne_bits(float x) {
     const uint32_t u = __float_as_uint(x);
     return (uint16_t)((u + 0x7FFFu + ((u >> 16) & 1u)) >> 16);
 }
+// bf16 pairs: the largest magnitudes of both halves (a not finite one is >= 0x7f80), and the
+// pair with its values that are not finite zeroed.
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+__device__ inline u16x2 bf16_top(u16x2 top, int x) {
+    return __builtin_elementwise_max(top, __builtin_bit_cast(u16x2, x & 0x7fff7fff));
+}
+__device__ inline bool bf16_not_finite(uint32_t h) { return (h & 0x7fffu) >= 0x7f80u; }
+__device__ inline int bf16_clean(int x) {
+    if (bf16_not_finite((uint32_t)x & 0xffffu)) x &= 0xffff0000;
+    if (bf16_not_finite((uint32_t)x >> 16)) x &= 0xffff;
+    return x;
+}
+__device__ inline float trunc_bf16(float x) { return __uint_as_float(__float_as_uint(x) & 0xffff0000u); }
 __device__ inline float bf16_bits_to_float(uint16_t b) { return __uint_as_float((uint32_t)b << 16); }
 
 // Interleaved waves (IW), as in the fp64 kernel: grid (nwg, Hkv), the eight waves of a
@@ -2405,14 +2425,31 @@ __device__ inline float bf16_bits_to_float(uint16_t b) { return __uint_as_float(
 // bf16 verify: 60.4 + 6.7 -> 59.7 + 4.9 us (stream + merge in the trace), traffic 1.149 ->
 // 1.025 x algorithmic. Every wave then holds the same rows, so the hi / lo split of Q is
 // shared: wave v splits step v and the eight steps go round through LDS (64.6 -> 63.1 us).
-constexpr int kBfRedRegion = 8192 + 32;  // o of the 32 hi-column lanes (8 rows x 256), then l
-constexpr int kBfRedO = 256 + 32;        // m [8 waves][8 rows] (floats), 8 bad flags
-__host__ __device__ constexpr size_t bf_iw_red_bytes() { return kBfRedO + 3 * (size_t)kBfRedRegion; }
+// WIDE: a region holds half of the dims of 16 rows, and the rounds run once per half.
+__host__ __device__ constexpr int bf_rows(bool wide) { return wide ? 16 : 8; }
+// a region: 8 KiB of o (8 rows x 256 dims, or 16 x 128), then l [row]
+__host__ __device__ constexpr int bf_red_region(bool wide) { return 8192 + 4 * bf_rows(wide); }
+// before the regions: m [8 waves][rows] (floats), 8 bad flags
+__host__ __device__ constexpr int bf_red_o(bool wide) { return 32 * bf_rows(wide) + 32; }
+__host__ __device__ constexpr size_t bf_iw_red_bytes(bool wide) {
+    return bf_red_o(wide) + 3 * (size_t)bf_red_region(wide);
+}
 
-template <int ADDR, bool IW = false>
+// A lane's offset in copy instruction j, for K and for V.
+__device__ inline uint32_t bf_copy_k(uint32_t ln, uint32_t j, uint32_t row_bytes) {
+    return (ln >> 5) * row_bytes + 16u * ((ln & 31) ^ (2 * j + (ln >> 5)));
+}
+__device__ inline uint32_t bf_copy_v(uint32_t ln, uint32_t j, uint32_t row_bytes) {
+    return (ln >> 5) * row_bytes + 16u * (((((ln & 31) >> 1) ^ (2 * j + (ln >> 5))) << 1) | (ln & 1));
+}
+
+template <int ADDR, bool IW = false, bool WIDE = false>
 __global__ __launch_bounds__(kMaxWaves * kSW) void stream_bf16_mfma_kernel(StreamArgs a) {
     constexpr int D = 256;
     static_assert(ADDR == kAddrPaged, "paged pools");
+    static_assert(IW || !WIDE, "16 rows: interleaved waves");
+    constexpr int kRows = bf_rows(WIDE);
+    constexpr int kBfRedRegion = bf_red_region(WIDE), kBfRedO = bf_red_o(WIDE);
     constexpr float kLog2e = 1.4426950408889634f;
     constexpr float kLn2 = 0.6931471805599453f;
     extern __shared__ int smem[];
@@ -2438,8 +2475,8 @@ __global__ __launch_bounds__(kMaxWaves * kSW) void stream_bf16_mfma_kernel(Strea
     const char* kbase = a.k_pool + (size_t)g * D * 2;
     const char* vbase = a.v_pool + (size_t)g * D * 2;
     const int grp = lane >> 4, l16 = lane & 15;
-    const int rr = l16 & 7;           // the row of this lane's column
-    const bool hi_col = l16 < 8;      // column holds the row's hi part (else its lo part)
+    const int rr = l16 & (kRows - 1);  // the row of this lane's column
+    const bool hi_col = WIDE || l16 < 8;  // column holds the row's hi part (else its lo part)
     const int bs_mask = (1 << a.bs_shift) - 1;
     const float sl2 = a.scale * kLog2e;
     char* sK = reinterpret_cast<char*>(smem) + mfma_stage_offset(B, false) + (size_t)wave * kBfStage;
@@ -2452,10 +2489,8 @@ __global__ __launch_bounds__(kMaxWaves * kSW) void stream_bf16_mfma_kernel(Strea
     uint32_t k_off[8], v_off[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-        const int r = 2 * j + (lane >> 5), p16 = lane & 31;
-        const uint32_t hb = (uint32_t)(lane >> 5) * row_bytes;
-        k_off[j] = hb + 16u * (uint32_t)(p16 ^ r);
-        v_off[j] = hb + 16u * (uint32_t)((((p16 >> 1) ^ r) << 1) | (p16 & 1));
+        k_off[j] = bf_copy_k(lane, j, row_bytes);
+        v_off[j] = bf_copy_v(lane, j, row_bytes);
     }
     // LDS operand addresses. K, 32-dim step c: token l16, 16-byte chunk (4c + grp) ^ l16 =
     // byte 512 l16 + 16 (grp ^ (l16 & 3)) + 64 ((c & 3) ^ (l16 >> 2)) + 256 (c >> 2).
@@ -2490,33 +2525,35 @@ __global__ __launch_bounds__(kMaxWaves * kSW) void stream_bf16_mfma_kernel(Strea
     auto finish = [&](int fs, bool fsingle, int frows, int nb, bool fbad) {
         // O^T hi + lo columns; the row sum over the four lane groups
         l = allreduce_hi<16>(l, OpSum());
+        if constexpr (!WIDE) {
 #pragma unroll
-        for (int u = 0; u < 16; ++u)
+            for (int u = 0; u < 16; ++u)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) o[u][r] += dpp<kRor8>(o[u][r]);
+                for (int r = 0; r < 4; ++r) o[u][r] += dpp<kRor8>(o[u][r]);
+        }
         if constexpr (IW) {
             // The waves' rows into wave 0's: the rows' common max, then the rescaled o (the
-            // 32 hi-column lanes, which hold the rows after the fold) and l summed. Uniform
+            // hi-column lanes, which hold the rows after the fold) and l summed. Uniform
             // branches: every wave meets the same barriers. The next piece's copies are in
             // flight, so the LDS accesses are untracked and the barriers wait for LDS only.
             if (nb > 1) {
                 uint32_t lo = lane;  // opaque: the addresses are formed here
                 asm volatile("" : "+v"(lo));
                 const uint32_t rm = lds_addr(red);  // m of [wave][row] (floats)
-                const uint32_t rbad = rm + 256;     // [wave] (ints)
-                const uint32_t rro = lo & 7;        // this lane's row
+                const uint32_t rbad = rm + 32 * kRows;   // [wave] (ints)
+                const uint32_t rro = lo & (kRows - 1);   // this lane's row
                 auto sync = [&]() {
                     __builtin_amdgcn_s_waitcnt(kLgkm0);
                     __builtin_amdgcn_s_barrier();
                     asm volatile("" ::: "memory");
                 };
-                if (lane < 8) lds_w32(rm + 32 * wave + 4 * lo, __float_as_int(m));  // row = lane
+                if (lane < kRows) lds_w32(rm + 4 * kRows * wave + 4 * lo, __float_as_int(m));  // row = lane
                 if (lane == 0) lds_w32(rbad + 4 * wave, fbad ? 1 : 0);
                 sync();
                 int mv[kMaxWaves], bv[kMaxWaves];
                 static_for<0, kMaxWaves>([&](auto V) {
                     constexpr int v = decltype(V)::value;
-                    mv[v] = lds_r32<32 * v>(rm + 4 * rro);
+                    mv[v] = lds_r32<4 * kRows * v>(rm + 4 * rro);
                     bv[v] = lds_r32<4 * v>(rbad + 0 * lo);
                 });
                 asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(mv[0]));
@@ -2535,61 +2572,76 @@ __global__ __launch_bounds__(kMaxWaves * kSW) void stream_bf16_mfma_kernel(Strea
 #pragma unroll
                 for (int u = 0; u < 16; ++u) o[u] *= f;
                 m = M;
-                // Region r: d-tile u of hi-column lane j = 8 grp + l16 at byte 16 (32 u + j),
-                // then l [row].
+                // Region r: d-tile u of hi-column lane j = 8 grp + l16 (WIDE: lane j) at byte
+                // 16 (32 u + j) (WIDE: 16 (64 u + j), eight d-tiles per pass), then l [row].
                 const uint32_t reg0 = lds_addr(red + kBfRedO);
-                const uint32_t jo = 16 * ((lo >> 4) * 8 + (lo & 7));
-                auto put = [&](int r) {
+                const uint32_t jo = WIDE ? 16 * lo : 16 * ((lo >> 4) * 8 + (lo & 7));
+                constexpr int kTile = WIDE ? 1024 : 512;
+                constexpr int kPassTiles = WIDE ? 8 : 16;
+                auto put = [&](auto P, int r) {
+                    constexpr int u0 = decltype(P)::value * kPassTiles;
                     const uint32_t rs = reg0 + r * kBfRedRegion;  // uniform
                     if (hi_col) {
 #pragma unroll
-                        for (int u = 0; u < 16; ++u) lds_w128(rs + jo + 512 * u, __builtin_bit_cast(i32x4, o[u]));
+                        for (int u = 0; u < kPassTiles; ++u)
+                            lds_w128(rs + jo + kTile * u, __builtin_bit_cast(i32x4, o[u0 + u]));
                     }
-                    if (lane < 8) lds_w32(rs + 8192 + 4 * lo, __float_as_int(l));
+                    if (u0 == 0 && lane < kRows) lds_w32(rs + 8192 + 4 * lo, __float_as_int(l));
                 };
-                auto add = [&](int r) {  // in two halves of eight reads
+                auto add = [&](auto P, int r) {  // eight reads at a time
+                    constexpr int u0 = decltype(P)::value * kPassTiles;
                     const uint32_t rs = reg0 + r * kBfRedRegion;  // uniform
                     if (hi_col) {
-                        static_for<0, 2>([&](auto H) {
+                        static_for<0, kPassTiles / 8>([&](auto H) {
                             constexpr int h = decltype(H)::value;
                             i32x4 v[8];
                             static_for<0, 8>([&](auto U) {
                                 constexpr int u = decltype(U)::value;
-                                v[u] = lds_b128<512 * (8 * h + u)>(rs + jo);
+                                v[u] = lds_b128<kTile * (8 * h + u)>(rs + jo);
                             });
                             asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(v[0]));
 #pragma unroll
                             for (int u = 0; u < 8; ++u) {
                                 asm volatile("" : "+v"(v[u]));
-                                o[8 * h + u] += __builtin_bit_cast(f32x4, v[u]);
+                                o[u0 + 8 * h + u] += __builtin_bit_cast(f32x4, v[u]);
                             }
                         });
                     }
-                    int lv = lds_r32<8192>(rs + 4 * rro);
-                    asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(lv));
-                    l += __int_as_float(lv);
+                    if constexpr (u0 == 0) {
+                        int lv = lds_r32<8192>(rs + 4 * rro);
+                        asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(lv));
+                        l += __int_as_float(lv);
+                    }
                 };
-                if (nb > 4) {  // waves 4-6 into 0-2 (regions 0-2), then every region read
-                    if (wave >= 4 && wave < 7) put(wave - 4);
+                static_for<0, 16 / kPassTiles>([&](auto P) {
+                    if constexpr (decltype(P)::value > 0) sync();  // region 1 read
+                    if (nb > 4) {  // waves 4-6 into 0-2 (regions 0-2), then every region read
+                        if (wave >= 4 && wave < 7) put(P, wave - 4);
+                        sync();
+                        if (wave < 3) add(P, wave);
+                        sync();
+                    }
+                    if (nb > 7) {  // wave 7 into 3 (region 0)
+                        if (wave == 7) put(P, 0);
+                        sync();
+                        if (wave == 3) add(P, 0);
+                    }
+                    if (nb > 2) {  // waves 2, 3 into 0, 1 (regions 2, 1; region 0 may still be read)
+                        if (wave == 2) put(P, 2);
+                        if (wave == 3) put(P, 1);
+                        sync();
+                        if (wave == 0) add(P, 2);
+                        if (wave == 1) add(P, 1);
+                    }
+                    if (wave == 1) put(P, 1);  // wave 1 into 0 (region 1, which wave 1 read last)
                     sync();
-                    if (wave < 3) add(wave);
-                    sync();
-                }
-                if (nb > 7) {  // wave 7 into 3 (region 0)
-                    if (wave == 7) put(0);
-                    sync();
-                    if (wave == 3) add(0);
-                }
-                if (nb > 2) {  // waves 2, 3 into 0, 1 (regions 2, 1; region 0 may still be read)
-                    if (wave == 2) put(2);
-                    if (wave == 3) put(1);
-                    sync();
-                    if (wave == 0) add(2);
-                    if (wave == 1) add(1);
-                }
-                if (wave == 1) put(1);  // wave 1 into 0 (region 1, which wave 1 read last)
-                sync();
-                if (wave == 0) add(1);
+                    if (wave == 0) add(P, 1);
+                });
+                if constexpr (WIDE) sync();  // region 1 read: Q's parts go there next
+            } else {
+                // every wave has read this piece's Q steps before the next piece's go to LDS
+                __builtin_amdgcn_s_barrier();
+                asm volatile("" ::: "memory");
             }
         }
         if (idle) {
@@ -2710,15 +2762,17 @@ __global__ __launch_bounds__(kMaxWaves * kSW) void stream_bf16_mfma_kernel(Strea
                 }
                 vpg = pg;
             }
+            uint32_t lo = lane;  // WIDE: the copy offsets are formed here, not kept in registers
+            if constexpr (WIDE) asm volatile("" : "+v"(lo));
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
                 // pairs past the piece re-read its last pair (masked)
                 const int tt = min(t + 2 * j, (tb - 1) & ~1);
                 const int pg = __builtin_amdgcn_readlane(vpg, (tt >> a.bs_shift) - pgbase);
                 const size_t off = (((size_t)pg << a.bs_shift) | (size_t)(tt & bs_mask)) * row_bytes;
-                __builtin_amdgcn_global_load_lds(uniform_ptr(kbase + off) + k_off[j],
+                __builtin_amdgcn_global_load_lds(uniform_ptr(kbase + off) + (WIDE ? bf_copy_k(lo, j, row_bytes) : k_off[j]),
                                                  (lds_void*)(sK + 2 * j * kBfRow), 16, 0, kCpolNT);
-                __builtin_amdgcn_global_load_lds(uniform_ptr(vbase + off) + v_off[j],
+                __builtin_amdgcn_global_load_lds(uniform_ptr(vbase + off) + (WIDE ? bf_copy_v(lo, j, row_bytes) : v_off[j]),
                                                  (lds_void*)(sV + 2 * j * kBfRow), 16, 0, kCpolNT);
             }
         };
@@ -2737,26 +2791,41 @@ __global__ __launch_bounds__(kMaxWaves * kSW) void stream_bf16_mfma_kernel(Strea
         // (column < 8) or lo part, zero for rows past `rows`.
         bf16x8 qreg[8];
         const bool qlive = rr < rows;
-        auto split = [&](const float4& q0, const float4& q1) {
+        // WIDE: part 0, 1 or 2 of the exact split (each the truncated rest, 3 x 8 bits)
+        auto split = [&](const float4& q0, const float4& q1, int part) {
             const float xv[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
             bf16x8 r;
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
                 const float x = qlive ? xv[e] : 0.f;
-                const uint16_t h = bf16_rne_bits(x);
-                const uint16_t b16 = hi_col ? h : bf16_rne_bits(x - bf16_bits_to_float(h));
+                uint16_t b16;
+                if constexpr (WIDE) {
+                    float rest = x;
+                    for (int i = 0; i < part; ++i) rest -= trunc_bf16(rest);
+                    b16 = (uint16_t)(__float_as_uint(rest) >> 16);
+                } else {
+                    const uint16_t h = bf16_rne_bits(x);
+                    b16 = hi_col ? h : bf16_rne_bits(x - bf16_bits_to_float(h));
+                }
                 r[e] = __builtin_bit_cast(__bf16, b16);
             }
             return r;
         };
         if constexpr (IW) {
             // Every wave holds the same rows: wave v splits step v into LDS (exchange region 0,
-            // which no finish uses between this barrier and the next piece's first one) and
-            // reads the eight steps back. The LDS accesses are untracked (copies in flight).
+            // WIDE: parts 1 and 2 into those regions, for the batches; no finish uses them between
+            // this barrier and the next piece's first one) and reads the eight steps back. The LDS accesses are untracked (copies in
+            // flight).
             uint32_t lo = lane;
             asm volatile("" : "+v"(lo));
             const uint32_t qst = lds_addr(red + kBfRedO) + 16 * lo;
-            lds_w128(qst + 1024 * wave, __builtin_bit_cast(i32x4, split(qstep[0], qstep[1])));
+            lds_w128(qst + 1024 * wave, __builtin_bit_cast(i32x4, split(qstep[0], qstep[1], 0)));
+            if constexpr (WIDE) {
+                lds_w128(qst + kBfRedRegion + 1024 * wave,
+                         __builtin_bit_cast(i32x4, split(qstep[0], qstep[1], 1)));
+                lds_w128(qst + 2 * kBfRedRegion + 1024 * wave,
+                         __builtin_bit_cast(i32x4, split(qstep[0], qstep[1], 2)));
+            }
             __builtin_amdgcn_s_waitcnt(kLgkm0);
             __builtin_amdgcn_s_barrier();
             asm volatile("" ::: "memory");
@@ -2773,7 +2842,7 @@ __global__ __launch_bounds__(kMaxWaves * kSW) void stream_bf16_mfma_kernel(Strea
             }
         } else {
 #pragma unroll
-            for (int c = 0; c < 8; ++c) qreg[c] = split(qraw[c][0], qraw[c][1]);
+            for (int c = 0; c < 8; ++c) qreg[c] = split(qraw[c][0], qraw[c][1], 0);
         }
         int it = 0;  // this wave's batch index in the piece
         for (int t = t1; t < tb; t += kStepT, ++it) {
@@ -2792,9 +2861,12 @@ __global__ __launch_bounds__(kMaxWaves * kSW) void stream_bf16_mfma_kernel(Strea
                 constexpr int c = decltype(C)::value;
                 kr[c] = lds_b128<256 * (c >> 2)>(k_addr[c & 3]);
             });
+            // WIDE: the sixteen V addresses are formed here, not kept in registers
+            int zo = z;
+            if constexpr (WIDE) asm volatile("" : "+v"(zo));
             static_for<0, 16>([&](auto U) {
                 constexpr int u = decltype(U)::value;
-                vr[u] = lds_tr16<0>(v_lane + ((uint32_t)(u ^ z) << 5));
+                vr[u] = lds_tr16<0>(v_lane + ((uint32_t)(u ^ zo) << 5));
             });
             asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(kr[0]), "+v"(kr[1]), "+v"(kr[2]), "+v"(kr[3]));
 #pragma unroll
@@ -2812,11 +2884,49 @@ __global__ __launch_bounds__(kMaxWaves * kSW) void stream_bf16_mfma_kernel(Strea
 #pragma unroll
             for (int c = 0; c < 8; ++c)
                 st = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, kr[c]), qreg[c], st, 0, 0, 0);
+            // Values that are not finite (WIDE): part 0 alone meets them in K (a zero part 1 or 2,
+            // or one of the other sign, would turn an infinite score into NaN), and no matrix
+            // product in V, where a row that masks the key has a zero weight.
+            bool v_odd = false;
+            if constexpr (WIDE) {
+                u16x2 top = {0, 0}, ktop = {0, 0};
+#pragma unroll
+                for (int i = 0; i < 16; ++i) top = bf16_top(bf16_top(top, vr[i][0]), vr[i][1]);
+#pragma unroll
+                for (int i = 0; i < 8; ++i)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) ktop = bf16_top(ktop, kr[i][j]);
+                v_odd = __any(top[0] >= 0x7f80 || top[1] >= 0x7f80);
+                if (__any(ktop[0] >= 0x7f80 || ktop[1] >= 0x7f80)) {
+#pragma unroll
+                    for (int i = 0; i < 8; ++i)
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) kr[i][j] = bf16_clean(kr[i][j]);
+                }
+                // Parts 1 and 2 stay in LDS (a finish writes the regions after its first
+                // barrier): in registers beside part 0 they spill.
+                const uint32_t ql = lds_addr(red + kBfRedO) + kBfRedRegion + 16 * lane;
+                static_for<0, 4>([&](auto H) {
+                    constexpr int part = decltype(H)::value >> 1, h = decltype(H)::value & 1;
+                    i32x4 qv[4];
+                    static_for<0, 4>([&](auto C) {
+                        constexpr int c = decltype(C)::value;
+                        qv[c] = lds_b128<part * kBfRedRegion + 1024 * (4 * h + c)>(ql);
+                    });
+                    asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(qv[0]));
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) {
+                        asm volatile("" : "+v"(qv[c]));
+                        st = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, kr[4 * h + c]),
+                                                                     __builtin_bit_cast(bf16x8, qv[c]), st, 0, 0, 0);
+                    }
+                });
+            }
             float sv[4];
             float mx = -INFINITY;
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const float full = st[r] + dpp<kRor8>(st[r]);
+                const float full = WIDE ? st[r] : st[r] + dpp<kRor8>(st[r]);
                 const int tok = t + 4 * grp + r;
                 const bool ok = row_live && tok >= ta && tok < tb && tok <= pq && tok >= wsr;
                 sv[r] = ok ? full * sl2 : -INFINITY;
@@ -2829,13 +2939,20 @@ __global__ __launch_bounds__(kMaxWaves * kSW) void stream_bf16_mfma_kernel(Strea
             const float alpha = move ? exp2f(m - m_new) : 1.f;  // m = -inf gives 0
             const float m_use = m_new == -INFINITY ? 0.f : m_new;
             float p[4];
-            s16x4 pb;
+            s16x4 pb, pmid, plo;  // pmid, plo: WIDE
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 p[r] = exp2f(sv[r] - m_use);  // masked: exp2(-inf) = 0
                 const uint32_t u = __float_as_uint(p[r]);
                 const uint16_t h = (uint16_t)(u >> 16);  // P_hi: p truncated to bf16
-                pb[r] = (short)(hi_col ? h : bf16_rne_bits(p[r] - __uint_as_float(u & 0xffff0000u)));
+                const float rest = p[r] - __uint_as_float(u & 0xffff0000u);
+                if constexpr (WIDE) {
+                    pb[r] = (short)h;
+                    pmid[r] = (short)(__float_as_uint(rest) >> 16);
+                    plo[r] = (short)(__float_as_uint(rest - trunc_bf16(rest)) >> 16);
+                } else {
+                    pb[r] = (short)(hi_col ? h : bf16_rne_bits(rest));
+                }
             }
             l = l * alpha + ((p[0] + p[1]) + (p[2] + p[3]));
             m = m_new;
@@ -2843,9 +2960,60 @@ __global__ __launch_bounds__(kMaxWaves * kSW) void stream_bf16_mfma_kernel(Strea
 #pragma unroll
                 for (int u = 0; u < 16; ++u) o[u] *= alpha;
             }
+            if constexpr (WIDE) {
+                if (v_odd) {
+                    // A row that attends such a key gets its value, found by products of
+                    // indicators (a weight of zero times it is NaN); then V without them.
+                    s16x4 b_live, b_zero;
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const int tok = t + 4 * grp + r;
+                        const bool ok = row_live && tok >= ta && tok < tb && tok <= pq && tok >= wsr;
+                        b_live[r] = ok && !(p[r] == 0.f) ? (short)0x3f80 : (short)0;
+                        b_zero[r] = ok && p[r] == 0.f ? (short)0x3f80 : (short)0;
+                    }
+#pragma unroll
+                    for (int u = 0; u < 16; ++u) {
+                        const s16x4 vh = __builtin_bit_cast(s16x4, vr[u]);
+                        s16x4 i_up, i_down, i_nan, i_any;
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            const uint32_t h = (uint16_t)vh[e];
+                            i_up[e] = h == 0x7f80u ? (short)0x3f80 : (short)0;
+                            i_down[e] = h == 0xff80u ? (short)0x3f80 : (short)0;
+                            i_nan[e] = (h & 0x7fffu) > 0x7f80u ? (short)0x3f80 : (short)0;
+                            i_any[e] = bf16_not_finite(h) ? (short)0x3f80 : (short)0;
+                        }
+                        const f32x4 none = {0.f, 0.f, 0.f, 0.f};
+                        const f32x4 up = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(i_up, b_live, none, 0, 0, 0);
+                        const f32x4 down = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(i_down, b_live, none, 0, 0, 0);
+                        const f32x4 nan1 = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(i_nan, b_live, none, 0, 0, 0);
+                        const f32x4 nan0 = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(i_any, b_zero, none, 0, 0, 0);
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            if (up[r] > 0.f) o[u][r] += INFINITY;
+                            if (down[r] > 0.f) o[u][r] -= INFINITY;
+                            if (nan1[r] + nan0[r] > 0.f) o[u][r] = __builtin_nanf("");
+                        }
+                        vr[u][0] = bf16_clean(vr[u][0]);
+                        vr[u][1] = bf16_clean(vr[u][1]);
+#if defined(__HIP_DEVICE_COMPILE__)
+                        asm volatile("" : "+v"(o[u]), "+v"(vr[u]));  // one d-tile at a time
+#endif
+                    }
+                }
+            }
 #pragma unroll
             for (int u = 0; u < 16; ++u)
                 o[u] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4, vr[u]), pb, o[u], 0, 0, 0);
+            if constexpr (WIDE) {
+#pragma unroll
+                for (int u = 0; u < 16; ++u)
+                    o[u] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4, vr[u]), pmid, o[u], 0, 0, 0);
+#pragma unroll
+                for (int u = 0; u < 16; ++u)
+                    o[u] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4, vr[u]), plo, o[u], 0, 0, 0);
+            }
         }
         bad = __any(bad);
         if constexpr (IW) {
@@ -3348,6 +3516,30 @@ int32_t launch_mfma(StreamArgs a, hipStream_t st) {
                            : launch_mfma_addr<D, RG, PKV_MFMA_TG, WPH, kAddrPaged>(a, st);
 }
 
+// Interleaved waves: grid (nwg, Hkv), eight waves per kv head.
+size_t bf_iw_lds(int batch, bool wide) {
+    return mfma_stage_offset(batch, false) + (size_t)kMaxWaves * kBfStage + bf_iw_red_bytes(wide);
+}
+template <bool WIDE>
+int32_t launch_bf16_iw(StreamArgs a, hipStream_t st) {
+    const size_t lds = bf_iw_lds(a.batch, WIDE);
+    const void* fn = reinterpret_cast<const void*>(&stream_bf16_mfma_kernel<kAddrPaged, true, WIDE>);
+    if (!reserve_lds(fn, (int)kMfmaLdsMax))
+        return fail(PKV_ERR_HIP, "pkv_attend: could not reserve the kernel's LDS");
+    const int slots = fill_workgroups(fn, kMaxWaves * kSW, lds);
+    if (slots <= 0) return fail(PKV_ERR_HIP, "pkv_attend: occupancy query failed");
+    a.nwg = slots / a.Hkv > 0 ? slots / a.Hkv : 1;
+    if (a.nwg > a.nwg_cap) a.nwg = a.nwg_cap;
+    if (a.nwg > 1) a.nwg &= ~1;  // whole pairs (key_split)
+    a.lead = PKV_LEAD_BF16_IW;
+    hipLaunchKernelGGL((stream_bf16_mfma_kernel<kAddrPaged, true, WIDE>), dim3(a.nwg, a.Hkv), dim3(kMaxWaves * kSW),
+                       lds, st, a);
+    if (hipGetLastError() != hipSuccess)
+        return fail(PKV_ERR_HIP, "pkv_attend: the attention launch failed");
+    launch_merge<256, float>(a, false, st);
+    return PKV_OK;
+}
+
 // bf16 pools, head_dim 256, 5..8 rows per kv head: the bf16 matrix cores (paged pools,
 // block_size >= 2: a copy pair lies in one block); else two vector waves of 4 rows.
 int32_t launch_bf16_mfma(StreamArgs a, hipStream_t st) {
@@ -3357,24 +3549,7 @@ int32_t launch_bf16_mfma(StreamArgs a, hipStream_t st) {
     if (lds > kMfmaLdsMax || a.keys || a.ring_size > 0 || a.bs_shift < 1 || a.nr.k_new)
         return launch_r<256, uint16_t, 4, 2>(a, st);
     // Interleaved waves (grid (nwg, Hkv), eight waves per kv head) where the batch's LDS fits.
-    const size_t lds_iw = mfma_stage_offset(a.batch, false) + (size_t)kMaxWaves * kBfStage + bf_iw_red_bytes();
-    if (lds_iw <= kMfmaLdsMax) {
-        const void* fn = reinterpret_cast<const void*>(&stream_bf16_mfma_kernel<kAddrPaged, true>);
-        if (!reserve_lds(fn, (int)kMfmaLdsMax))
-            return fail(PKV_ERR_HIP, "pkv_attend: could not reserve the kernel's LDS");
-        const int slots = fill_workgroups(fn, kMaxWaves * kSW, lds_iw);
-        if (slots <= 0) return fail(PKV_ERR_HIP, "pkv_attend: occupancy query failed");
-        a.nwg = slots / a.Hkv > 0 ? slots / a.Hkv : 1;
-        if (a.nwg > a.nwg_cap) a.nwg = a.nwg_cap;
-        if (a.nwg > 1) a.nwg &= ~1;  // whole pairs (key_split)
-        a.lead = PKV_LEAD_BF16_IW;
-        hipLaunchKernelGGL((stream_bf16_mfma_kernel<kAddrPaged, true>), dim3(a.nwg, a.Hkv), dim3(kMaxWaves * kSW),
-                           lds_iw, st, a);
-        if (hipGetLastError() != hipSuccess)
-            return fail(PKV_ERR_HIP, "pkv_attend: the attention launch failed");
-        launch_merge<256, float>(a, false, st);
-        return PKV_OK;
-    }
+    if (bf_iw_lds(a.batch, false) <= kMfmaLdsMax) return launch_bf16_iw<false>(a, st);
     const void* fn = reinterpret_cast<const void*>(&stream_bf16_mfma_kernel<kAddrPaged>);
     if (!reserve_lds(fn, (int)kMfmaLdsMax))
         return fail(PKV_ERR_HIP, "pkv_attend: could not reserve the kernel's LDS");
@@ -3426,6 +3601,11 @@ int32_t launch_rows_addr(StreamArgs a, hipStream_t st) {
 template <int D>
 int32_t launch_many_rows(StreamArgs a, int rows, hipStream_t st) {
     return rows <= 16 ? launch_rows_addr<D, 1>(a, st) : launch_rows_addr<D, 2>(a, st);
+}
+// Whether bf16 pools take up to 16 rows in one launch: stream_bf16_mfma_kernel's addressing
+// (paged, blocks of two tokens at least) and its LDS at this batch.
+bool bf16_wide_fits(const StreamArgs& a, int D) {
+    return D == 256 && !a.keys && a.ring_size == 0 && a.bs_shift >= 1 && bf_iw_lds(a.batch, true) <= kMfmaLdsMax;
 }
 // Whether a launch of up to kRowsMax rows fits the CU's LDS at this batch.
 bool many_rows_fit(int D, int batch, int rows) {
@@ -3557,13 +3737,17 @@ int32_t stream_attend(const pkv_params* p, const float* q, const void* k_pool,
         const int per = q_len < kRowsMax / G ? q_len : kRowsMax / G;
         if (many_rows_fit(p->head_dim, batch, G * per)) per_launch = per;
     }
+    // bf16 pools: groups of up to 16 rows (10 rows: the step of 16 sequences 106.4 -> 85.2 us
+    // against groups of 8).
+    if (bf16 && G * q_len > 8 && bf16_wide_fits(a, p->head_dim)) per_launch = q_len < 16 / G ? q_len : 16 / G;
     for (int j0 = 0; j0 < q_len; j0 += per_launch) {
         a.j0 = j0;
         a.q_cnt = q_len - j0 < per_launch ? q_len - j0 : per_launch;
         a.rows_seq = p->num_heads * a.q_cnt;
         const int rows = G * a.q_cnt;
-        if (rows > 8) {  // fp32 pools
-            const int32_t rc = p->head_dim == 256 ? launch_many_rows<256>(a, rows, st) : launch_many_rows<512>(a, rows, st);
+        if (rows > 8) {
+            const int32_t rc = bf16 ? launch_bf16_iw<true>(a, st)
+                               : p->head_dim == 256 ? launch_many_rows<256>(a, rows, st) : launch_many_rows<512>(a, rows, st);
             if (rc != PKV_OK) return rc;
             continue;
         }

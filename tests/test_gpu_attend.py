@@ -290,6 +290,36 @@ def test_verify_bf16_mfma(gpu, hq, hkv, q_len, bs, window):
     _batched_case(rng, ctx.size, q_len, ctx, hq, hkv, 256, bs, window, BF16, 0.0625)
 
 
+@pytest.mark.parametrize("hq,hkv,q_len,bs,window", [
+    (16, 8, 5, 16, 0),     # the engine's verify: 10 rows
+    (16, 8, 8, 16, 1024),  # 16 rows, every column used
+    (16, 8, 9, 16, 0),     # 16 rows, then a group of 2
+    (16, 16, 9, 16, 0),    # 9 rows at G = 1
+    (16, 16, 16, 16, 40),  # 16 rows at G = 1
+    (12, 4, 4, 16, 0),     # G = 3: 12 rows
+    (16, 2, 2, 2, 0),      # G = 8, smallest block size the kernel takes
+    (16, 4, 3, 64, 33),    # G = 4: 12 rows, large blocks, an odd window
+    (16, 8, 5, 1, 0),      # blocks of one token: groups of 8 rows on the vector kernel
+], ids=["q5", "rows16", "q9", "g1-q9", "g1-q16", "g3", "g8-bs2", "g4-w33", "bs1"])
+def test_verify_bf16_wide(gpu, hq, hkv, q_len, bs, window):
+    """bf16 pools with 9..16 query rows per kv head in one pass over the keys (a column of
+    the matrix product per row): pieces of one batch, of two to eight and of many, odd and
+    even first and last keys, against the oracle on the same bf16 values (2e-2)."""
+    print(f"[attend] bf16 wide {hq}q/{hkv}kv q_len {q_len} bs {bs} window {window}", flush=True)
+    rng = np.random.default_rng(hq * 100 + hkv * 10 + q_len + bs + window)
+    ctx = np.concatenate([[0, 1, 2, 3, 11, 16, 17, 31, 60, 75, 107, 121], rng.integers(40, 5000, 7)])
+    _batched_case(rng, ctx.size, q_len, ctx, hq, hkv, 256, bs, window, BF16, 0.0625)
+
+
+@pytest.mark.parametrize("batch", [300, 512])
+def test_bf16_wide_large_batch(gpu, batch):
+    """10 rows per kv head at 300 sequences (the wide form's LDS holds their ints) and at 512
+    (it no longer does: groups of 8 rows)."""
+    print(f"[attend] bf16 wide, batch {batch}", flush=True)
+    rng = np.random.default_rng(batch)
+    _batched_case(rng, batch, 5, rng.integers(1, 300, batch), 16, 8, 256, 16, 0, BF16, 0.0625)
+
+
 @pytest.mark.parametrize("q_len", [1, 4], ids=["decode-vector", "verify-mfma"])
 def test_batch_4096_large_lds(gpu, q_len):
     """The largest batch pkv_attend takes: the stream kernels keep 5 ints per sequence in

@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 
 from oracle import oracle as O
-from pkv import F32, LayerSpec, hip, lib
+from pkv import BF16, F32, LayerSpec, hip, lib
 from pkv.engine import make_params
 from tests import parity
 from tests.test_gpu_attend import _batched_case
@@ -108,3 +108,39 @@ def test_rows_masked_values_not_finite(gpu, hq, hkv, d, q_len, value):
     assert np.array_equal(last[..., 4:d - 1], clean[:, -1][..., 4:d - 1])
     want = np.full(last[..., [3, d - 1]].shape, value, np.float32)
     assert np.array_equal(last[..., [3, d - 1]], want, equal_nan=True)
+
+
+@pytest.mark.parametrize("hq,hkv,q_len", [(16, 8, 5), (16, 16, 16)])
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan])
+def test_bf16_wide_values_not_finite(gpu, hq, hkv, q_len, value):
+    # bf16 pools, 9..16 rows: a V value that is not finite reaches the rows that attend its
+    # key and no other; a K value of -inf gives the key no weight, as a very negative one.
+    print(f"[rows] bf16, {value} in a masked key, {hq}q/{hkv}kv q_len {q_len}", flush=True)
+    rng = np.random.default_rng(9)
+    bs, d, nblk, pos = 16, 256, 20, np.array([70, 29, 300], np.int32)
+    tables = rng.permutation(3 * nblk).astype(np.int32).reshape(3, nblk)
+    k = O.to_bf16(rng.standard_normal((3 * nblk, bs, hkv, d), dtype=np.float32))
+    v = O.to_bf16(rng.standard_normal((3 * nblk, bs, hkv, d), dtype=np.float32))
+    q = rng.standard_normal((3, q_len, hq, d), dtype=np.float32)
+    q[..., 5] = np.abs(q[..., 5]) + 0.01
+    q[..., 6] = 1.0  # parts 1 and 2 are zero
+    p = make_params(LayerSpec(hq, hkv, d, 0, BF16), bs, 3 * nblk, 0.0625)
+    bits = O.to_bf16(np.full(1, value, np.float32))[0]
+    low, inf = (O.to_bf16(np.full(1, x, np.float32))[0] for x in (-1e30, -np.inf))
+    clean = _call("pkv_attend", p, q, k, v, tables, pos)
+    odd = v.copy()
+    for s in range(3):
+        t = int(pos[s]) + q_len - 1
+        odd[tables[s, t // bs], t % bs][:, [3, d - 1]] = bits
+    got = _call("pkv_attend", p, q, k, odd, tables, pos)
+    assert np.array_equal(got[:, :-1], clean[:, :-1])
+    last = got[:, -1]
+    assert np.array_equal(last[..., 4:d - 1], clean[:, -1][..., 4:d - 1])
+    want = np.full(last[..., [3, d - 1]].shape, value, np.float32)
+    assert np.array_equal(last[..., [3, d - 1]], want, equal_nan=True)
+    for dim in (5, 6):
+        k1, k2 = k.copy(), k.copy()
+        for s in range(3):
+            k1[tables[s, 1], 4][:, dim], k2[tables[s, 1], 4][:, dim] = low, inf
+        a, b = (_call("pkv_attend", p, q, x, v, tables, pos) for x in (k1, k2))
+        assert np.all(np.isfinite(b)) and np.array_equal(a, b)
