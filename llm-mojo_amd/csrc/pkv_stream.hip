@@ -2376,7 +2376,7 @@ __global__ __launch_bounds__(kMaxWaves * kSW, 2) void stream_rows_kernel(StreamA
 // (5.3 TB/s in the trace), so one pass instead of two halves the time of the second group, and
 // the third part costs nothing: 16 sequences of 512..4096 keys, 1..5 tokens at G = 2,
 // 60.5 + 4.7 (8 rows) + 20.6 + 5.3 us (2 rows) -> 62 + 5.0 us; error against
-// 64 bits 5.0e-6 -> 5.0e-7.
+// 64 bits 5.0e-6 -> 5.4e-7.
 // LDS per wave: K and V of 16 tokens, rows of 512 bytes; K's 16-byte chunk c of token r
 // sits at c ^ r and V's 32-byte chunk c at c ^ r, so the operand reads land on distinct
 // banks. A copy instruction moves two tokens (1 KiB): the batches start on even positions
@@ -3737,7 +3737,7 @@ int32_t stream_attend(const pkv_params* p, const float* q, const void* k_pool,
         const int per = q_len < kRowsMax / G ? q_len : kRowsMax / G;
         if (many_rows_fit(p->head_dim, batch, G * per)) per_launch = per;
     }
-    // bf16 pools: groups of up to 16 rows (10 rows: the step of 16 sequences 106.4 -> 85.2 us
+    // bf16 pools: groups of up to 16 rows (10 rows: the step of 16 sequences 106.2 -> 83.7 us
     // against groups of 8).
     if (bf16 && G * q_len > 8 && bf16_wide_fits(a, p->head_dim)) per_launch = q_len < 16 / G ? q_len : 16 / G;
     for (int j0 = 0; j0 < q_len; j0 += per_launch) {
