@@ -240,8 +240,8 @@ __global__ __launch_bounds__(kNT) void prefill_kernel(PrefillArgs a) {
     // table entry is one load per wave and tile (the same address in every lane), made a
     // step before the copies that use it; a copy's address is that block's first row
     // (scalar) plus a per-lane offset that is the same for every tile. Keys outside
-    // [k_lo, k_hi] (and tiles past the last) read rows of a valid block and are masked or
-    // never read; a bad entry reads block 0 (the whole range was checked up front).
+    // [k_lo, k_hi] (and tiles past the last) read rows of a valid block and are masked (their
+    // V rows zeroed, clean_v) or never read; a bad entry reads block 0 (the whole range was checked up front).
     // K: lane i loads the global chunk that belongs at 16-byte position i % 32 of its row,
     // i.e. chunk (i % 32) ^ (key & 15). V: LDS position p of key row k holds global chunk
     // 2 * ((p / 2) ^ (k & 15)) + p % 2 (the 32-byte chunk swizzle).
@@ -472,13 +472,37 @@ __global__ __launch_bounds__(kNT) void prefill_kernel(PrefillArgs a) {
     // LDS one step before its first reader. Copies past the last tile re-read valid rows
     // into buffers nobody reads again. The barriers carry no fence (a fence would wait for
     // the copies just issued).
-    auto step_barrier = [&]() {
+    auto step_wait = [&]() {
         asm volatile("s_waitcnt vmcnt(4)"
                      : "+v"(blk[0]), "+v"(blk[1])
                      :
                      : "memory");
+    };
+    auto step_join = [&]() {
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
+    };
+    auto step_barrier = [&]() {
+        step_wait();
+        step_join();
+    };
+    // Between the wait for a wave's V rows of tile t and the barrier behind which they are first
+    // read: rows outside the range's keys may hold anything and are zeroed, so that a value that
+    // is not finite cannot meet a zero weight. (Untracked writes: copies are in flight.)
+    auto clean_v = [&](auto PAR, int t) {
+        const int kb = kb0 + t * kKT + 8 * wave;
+        if (kb < k_lo || kb + 7 > k_hi) {
+            uint32_t ln = lane;  // opaque: the addresses are formed here, not kept in registers
+            asm volatile("" : "+v"(ln));
+            const uint32_t dst = lds_addr(sV[0]) + decltype(PAR)::value * 2 * kVTile + 512 * 8 * wave + 16 * ln;
+            const i32x4 zero = {0, 0, 0, 0};
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int key = kb + 2 * j + (int)(ln >> 5);
+                if (key < k_lo || key > k_hi) asm volatile("ds_write_b128 %0, %1" ::"v"(dst + 1024 * j), "v"(zero) : "memory");
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        }
     };
     constexpr int kLead = 4;
     if (wave < kLead) {
@@ -486,7 +510,9 @@ __global__ __launch_bounds__(kNT) void prefill_kernel(PrefillArgs a) {
             constexpr int par = decltype(PAR)::value;
             issue_k(Par<par ^ 1>{}, t + 1, blk[par ^ 1]);  // step 2t
             score(PAR, t);
-            step_barrier();
+            step_wait();
+            clean_v(PAR, t);
+            step_join();
             load_blk_async(t + 2, blk[par]);  // step 2t + 1
             issue_v(Par<par ^ 1>{}, t + 1, blk[par ^ 1]);
             accumulate(PAR);
@@ -498,7 +524,9 @@ __global__ __launch_bounds__(kNT) void prefill_kernel(PrefillArgs a) {
         }
     } else {
         issue_k(Par<1>{}, 1, blk[1]);  // step 0
-        step_barrier();
+        step_wait();
+        clean_v(Par<0>{}, 0);
+        step_join();
         auto trail = [&](auto PAR, int t) {
             constexpr int par = decltype(PAR)::value;
             load_blk_async(t + 2, blk[par]);  // step 2t + 1
@@ -507,7 +535,11 @@ __global__ __launch_bounds__(kNT) void prefill_kernel(PrefillArgs a) {
             step_barrier();
             issue_k(PAR, t + 2, blk[par]);  // step 2t + 2
             accumulate(PAR);
-            if (t + 1 < ntiles) step_barrier();
+            if (t + 1 < ntiles) {
+                step_wait();
+                clean_v(Par<par ^ 1>{}, t + 1);
+                step_join();
+            }
         };
         for (int t = 0; t < ntiles; t += 2) {
             trail(Par<0>{}, t);
@@ -677,11 +709,18 @@ __global__ __launch_bounds__(kNT) void prefill_split_kernel(PrefillArgs a) {
     // aligned to 512: c and u flip address bits.)
     for (int t = t1; t <= k_hi; t += kStep) {
         asm volatile("s_waitcnt vmcnt(0)" : "+v"(ent) : : "memory");  // the batch is in LDS
-        if (t + kBT - 1 > k_hi) {
-            // Rows past the range's last key may hold anything: V's are zeroed, so that a value
-            // that is not finite cannot meet a zero weight.
-            for (int r = k_hi + 1 - t; r < kBT; ++r)
-                if (lane < 32) *reinterpret_cast<uint4*>(sV + r * kD + 8 * lane) = make_uint4(0, 0, 0, 0);
+        if (t < k_lo || t + kBT - 1 > k_hi) {
+            // Rows outside the range's keys may hold anything (a batch before k_lo too: its rows
+            // may come from the range's first block): V's are zeroed, so that a value that is
+            // not finite cannot meet a zero weight.
+            const uint32_t ln = opaque_lane();
+            const uint32_t dst = lds_addr(sV) + 16 * ln;
+            const i32x4 zero = {0, 0, 0, 0};
+#pragma unroll
+            for (int j = 0; j < kBT / 2; ++j) {
+                const int key = t + 2 * j + (int)(ln >> 5);
+                if (key < k_lo || key > k_hi) asm volatile("ds_write_b128 %0, %1" ::"v"(dst + 1024 * j), "v"(zero) : "memory");
+            }
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         }
         f32x4 st[RT];

@@ -2,7 +2,8 @@
 workgroup, the keys shared out over its waves) against the oracle, at the edges of its query
 tiles (one query; a tile, a tile and one; the largest 16-row and the smallest and largest
 32-row grids of one sequence), with fewer batches of keys than waves, windows, block sizes and
-ragged counts; bad tables, inactive sequences and unwritten pool rows that are not finite.
+ragged counts; bad tables, inactive sequences and, with the 128-row kernel beside it, pool rows
+outside the attended keys that are not finite.
 Same tolerance as the other prefill tests (2e-2, tests/parity.py)."""
 import ctypes
 
@@ -71,3 +72,29 @@ def test_prefill_split_contract_and_unwritten_rows(gpu, n):
     bad = tables.copy()
     bad[0, 1] = nb
     assert np.all(np.isnan(call(bad, pos, 600)))                # an entry outside the pool
+
+
+@pytest.mark.parametrize("batch", [1, 40], ids=["16-rows", "128-rows"])
+@pytest.mark.parametrize("bs,window,pos,n", [
+    (8, 4, 13, 1), (8, 4, 14, 3), (8, 0, 13, 1), (16, 5, 20, 1), (16, 0, 3, 2), (64, 20, 100, 9), (8, 70, 150, 5),
+])
+def test_prefill_rows_outside_the_range(gpu, batch, bs, window, pos, n):
+    # Every pool row but those of the keys the queries attend is NaN in V: the copies round
+    # the range down and up to whole batches and tiles, in the rows of its first and last block.
+    print(f"[prefill split] NaN outside the keys, batch {batch} bs {bs} window {window} pos {pos}", flush=True)
+    rng = np.random.default_rng(bs + pos)
+    hq, hkv, d = 16, 8, 256
+    stride = (pos + n + bs - 1) // bs + 1
+    p = make_params(LayerSpec(hq, hkv, d, window=window, kv_dtype=BF16), bs, batch * stride, 0.0625)
+    tables = rng.permutation(batch * stride).astype(np.int32).reshape(batch, stride)
+    v = np.full((batch * stride, bs, hkv * d), 0x7FC0, np.uint16)
+    for t in range(max(0, pos - window + 1) if window else 0, pos + n):
+        v[tables[:, t // bs], t % bs] = 0x3F80  # 1.0
+    q = hip.DeviceArray.from_numpy(O.to_bf16(rng.standard_normal((batch * n, hq, d), dtype=np.float32)))
+    k, out = hip.DeviceArray(v.shape, np.uint16, zero=True), hip.DeviceArray((batch * n, hq, d), np.float32)
+    dv, dt = hip.DeviceArray.from_numpy(v), hip.DeviceArray.from_numpy(tables)
+    dp = hip.DeviceArray.from_numpy(np.full(batch, pos, np.int32))
+    off = hip.DeviceArray.from_numpy((np.arange(batch + 1) * n).astype(np.int32))
+    lib.call("pkv_prefill", None, ctypes.byref(p), q.ptr, k.ptr, dv.ptr, dt.ptr, stride, dp.ptr, off.ptr, n, batch,
+             1000, out.ptr)
+    assert np.allclose(out.numpy(), 1.0, atol=1e-6)  # equal weights of rows of ones
