@@ -931,13 +931,19 @@ int32_t pkv_prefill(void* stream, const pkv_params* p, const void* q, const void
     // never pays against one of the next (16q/8kv/256, 3000 cached tokens, one sequence:
     // 256 new tokens 111.8 (128 rows) / 66.6 (32) / 49.9 us (16); 512: 123.5 / 76.6 / 99.6;
     // 1024: 147.6 / 155.6 / 215.3).
+    // Few keys leave the waves nothing to share out, and the combination is all that is added:
+    // without a prefix 8 tokens take 6.3 (128 rows) against 6.9 us (16), 33 take 8.6 against 7.0;
+    // 8 sequences of 33 tokens 9.1 against 10.9 us (32), 4 of 100 11.1 against 12.3, 2 of 130 12.4
+    // against 12.1. So 16 rows from 33 rows or 81 keys on (one 64-key tile and a block of slack
+    // in the caller's bound), 32 rows from 129 keys on.
     const void* split_fn = G == 1   ? reinterpret_cast<const void*>(&prefill_split_kernel<1, 2>)
                            : G == 2 ? reinterpret_cast<const void*>(&prefill_split_kernel<2, 2>)
                                     : reinterpret_cast<const void*>(&prefill_split_kernel<4, 2>);
     const int resident = device_fill_workgroups(split_fn, kNT, 0, INT32_MAX);
     if (resident <= 0) return fail(PKV_ERR_HIP, "pkv_prefill: occupancy query failed");
-    auto workgroups = [&](int64_t r) { return ((int64_t)max_q * G + r - 1) / r * p->num_kv_heads * batch; };
-    const int rows = workgroups(16) <= resident ? 16 : (workgroups(32) <= resident ? 32 : 128);
+    const int64_t total_rows = (int64_t)max_q * G;
+    auto fits = [&](int64_t r) { return (total_rows + r - 1) / r * p->num_kv_heads * batch <= resident; };
+    const int rows = fits(16) && (total_rows > 32 || max_pos >= 80) ? 16 : (fits(32) && max_pos >= 128 ? 32 : 128);
     const int qb = rows / G;
     a.qtiles = (int)(((int64_t)max_q + qb - 1) / qb);
     // one workgroup id per (sequence, tile, kv head); the launch's work-items must fit in 32 bits
