@@ -1249,8 +1249,8 @@ __host__ __device__ constexpr size_t iw_red_bytes() { return kRedO + 4 * (size_t
 
 // FUSED: the launch of a fused append (paged pools); a separate instance, so the scalar
 // state of the appended rows costs the other launches nothing.
-template <int D, int RG, int TG, int WPH, int ADDR, bool FUSED, bool IW = false>
-__global__ __launch_bounds__(kMaxWaves * kSW) void stream_mfma_kernel(StreamArgs a) {
+template <int D, int RG, int TG, int WPH, int ADDR, bool FUSED, bool IW>
+__device__ __forceinline__ void mfma_workgroup(const StreamArgs& a) {
     constexpr int NQ = D / 64;  // 64-d chunks of a row
     constexpr int kSlot = mfma_slot(D);
     constexpr int U = 4 * TG;  // tokens per batch
@@ -1873,6 +1873,11 @@ __global__ __launch_bounds__(kMaxWaves * kSW) void stream_mfma_kernel(StreamArgs
     }
 }
 
+template <int D, int RG, int TG, int WPH, int ADDR, bool FUSED, bool IW = false>
+__global__ __launch_bounds__(kMaxWaves * kSW) void stream_mfma_kernel(StreamArgs a) {
+    mfma_workgroup<D, RG, TG, WPH, ADDR, FUSED, IW>(a);
+}
+
 // ---- fp64 MFMA path, 9..32 query rows per KV head: fp32 pools, head_dim 256 or 512 --------
 //
 // A verify of the engine's 5 tokens is 10 rows per kv head on the sliding layers and 40 on
@@ -1922,7 +1927,7 @@ typedef float f32x2v __attribute__((ext_vector_type(2)));
 typedef float f32x4v __attribute__((ext_vector_type(4)));
 
 template <int D, int RT, int ADDR>
-__global__ __launch_bounds__(kMaxWaves * kSW, 2) void stream_rows_kernel(StreamArgs a) {
+__device__ __forceinline__ void rows_workgroup(const StreamArgs& a) {
     constexpr bool RING = ADDR == kAddrRing;
     constexpr bool PAGED = ADDR == kAddrPaged;
     constexpr int NW = kMaxWaves;
@@ -2346,6 +2351,29 @@ __global__ __launch_bounds__(kMaxWaves * kSW, 2) void stream_rows_kernel(StreamA
         if (RT == 1 || nt <= 1) piece(std::integral_constant<int, 1>{});
         else piece(std::integral_constant<int, RT>{});
     }
+}
+
+template <int D, int RT, int ADDR>
+__global__ __launch_bounds__(kMaxWaves * kSW, 2) void stream_rows_kernel(StreamArgs a) {
+    rows_workgroup<D, RT, ADDR>(a);
+}
+
+// The same for a verify step that may bring no such sequence (head_dim 256): when none has more
+// than 8 rows in this launch, the workgroup runs the 8-row kernel's interleaved form, whose
+// products waste no matrix rows. Both take the grid, the workspace rows and the merge of the
+// larger group, and one wave's look at the query counts decides. Steps with room for 5 tokens
+// of 16q/8kv/256, GPU time of rows alone -> this, by the sequences that bring 5 (the others
+// 1..4): none of 32 x 1024 keys 121 -> 96 us, of 64 x 1024 226 -> 196 (in groups of 8 rows 100
+// and 190); a tenth 121 -> 121 and 227 -> 225 (117 and 210); all 121 -> 121 and 230 -> 230.
+template <int RT, int ADDR>
+__global__ __launch_bounds__(kMaxWaves * kSW, 2) void stream_verify_kernel(StreamArgs a) {
+    bool many = false;
+    for (int i = threadIdx.x & (kSW - 1); i < a.batch; i += kSW) {
+        const int n = a.q_lens[i];
+        many = many || (n <= a.q_len && a.G * min(n - a.j0, a.q_cnt) > 8);
+    }
+    if (__any(many)) rows_workgroup<256, RT, ADDR>(a);
+    else mfma_workgroup<256, 2, 1, 1, ADDR, false, true>(a);
 }
 
 // ---- bf16 MFMA path: bf16 pools, head_dim 256, 5..16 query rows per KV head ------------
@@ -3420,12 +3448,14 @@ constexpr size_t kMfmaLdsMax = kStreamLdsMax;
 // Interleaved waves (head_dim 256, paged or ring pools): grid (nwg, Hkv), eight waves per
 // kv head. False when the batch's LDS does not fit it (the caller then takes the launch
 // below).
+size_t mfma_iw_lds(int batch, bool fused) {
+    return mfma_stage_offset(batch, fused) + (size_t)kMaxWaves * mfma_stage_bytes(256, 1) + iw_red_bytes();
+}
 template <int ADDR>
 bool launch_mfma_iw(StreamArgs& a, hipStream_t st, int32_t* rc) {
     constexpr int D = 256, RG = 2, TG = 1;
     const bool fused = ADDR == kAddrPaged && a.nr.k_new && a.j0 == 0;
-    const size_t lds = mfma_stage_offset(a.batch, fused) + (size_t)kMaxWaves * mfma_stage_bytes(D, TG) +
-                       iw_red_bytes();
+    const size_t lds = mfma_iw_lds(a.batch, fused);
     if (lds > kMfmaLdsMax) return false;
     constexpr bool kFusable = ADDR == kAddrPaged;
     const void* fn = fused ? reinterpret_cast<const void*>(&stream_mfma_kernel<D, RG, TG, 1, ADDR, kFusable, true>)
@@ -3573,10 +3603,24 @@ int32_t launch_bf16_mfma(StreamArgs a, hipStream_t st) {
 #define PKV_LEAD_ROWS 64
 #endif
 constexpr int kRowsMax = 32;
+// Keys x kv heads of a step from which stream_verify_kernel looks at the query counts. Below, rows
+// of all sizes take less on stream_rows_kernel than in groups of 8 (8 x 512 keys, 1..4 tokens each:
+// 28 against 31 us), and the look costs a round trip (2 x 256 keys 15.4 -> 16.1 us).
+constexpr int64_t kVerifyLook = 8 * 8192;
 template <int D, int RT, int ADDR>
 int32_t launch_rows_kernel(StreamArgs a, hipStream_t st) {
-    const size_t lds = rows_lds(D, a.batch, RT);
-    const void* fn = reinterpret_cast<const void*>(&stream_rows_kernel<D, RT, ADDR>);
+    size_t lds = rows_lds(D, a.batch, RT);
+    auto kernel = &stream_rows_kernel<D, RT, ADDR>;
+    if constexpr (D == 256) {
+        const int64_t span = a.window > 0 ? (int64_t)a.window + a.q_cnt - 1 : INT64_MAX;
+        const int64_t keys = (int64_t)a.max_pos + 1 < span ? (int64_t)a.max_pos + 1 : span;
+        const size_t lds_iw = mfma_iw_lds(a.batch, false);
+        if (a.q_lens && keys * a.batch * a.Hkv >= kVerifyLook && lds_iw <= kMfmaLdsMax) {
+            kernel = &stream_verify_kernel<RT, ADDR>;
+            lds = lds > lds_iw ? lds : lds_iw;
+        }
+    }
+    const void* fn = reinterpret_cast<const void*>(kernel);
     if (lds > 64 * 1024 && !reserve_lds(fn, (int)kStreamLdsMax))
         return fail(PKV_ERR_HIP, "pkv_attend: could not reserve the kernel's LDS");
     const int slots = fill_workgroups(fn, kMaxWaves * kSW, lds);
@@ -3587,7 +3631,7 @@ int32_t launch_rows_kernel(StreamArgs a, hipStream_t st) {
     // the weighted units of the split must fit an int
     a.weighted = (int64_t)a.batch * (((int64_t)a.max_pos + 1) * 7 + PKV_LEAD_ROWS) <= INT32_MAX ? 1 : 0;
     a.lead = PKV_LEAD_ROWS;
-    hipLaunchKernelGGL((stream_rows_kernel<D, RT, ADDR>), dim3(a.nwg, a.Hkv), dim3(kMaxWaves * kSW), lds, st, a);
+    hipLaunchKernelGGL(kernel, dim3(a.nwg, a.Hkv), dim3(kMaxWaves * kSW), lds, st, a);
     if (hipGetLastError() != hipSuccess)
         return fail(PKV_ERR_HIP, "pkv_attend: the attention launch failed");
     launch_merge<D, double>(a, false, st);

@@ -84,6 +84,60 @@ def test_rows_ring(gpu, hq, hkv, d, q_len):
                  O.attend_f64(q, paged[0].ravel(), paged[1].ravel(), tables, pos, *args, scale=0.0625))
 
 
+@pytest.mark.parametrize("hq,hkv,q_len,window,ring", [
+    (16, 8, 5, 0, 0), (16, 8, 5, 200, 208), (16, 16, 16, 100, 0), (12, 4, 3, 0, 0), (16, 8, 18, 0, 0),
+    (16, 8, 16, 200, 216),
+])
+@pytest.mark.parametrize("many", [False, True], ids=["few", "many"])
+def test_verify_large_step_by_counts(gpu, hq, hkv, q_len, window, ring, many):
+    # A step whose bound on the keys is large (stream_verify_kernel: 65536 keys times kv heads): no
+    # sequence with more than 8 rows, or two; sequences without queries, inactive ones and invalid
+    # counts among them.
+    print(f"[rows] counts {hq}q/{hkv}kv q_len {q_len} window {window} ring {ring} many {many}", flush=True)
+    rng = np.random.default_rng(hq + q_len + window + many)
+    d, bs, few = 256, 16, 8 * hkv // hq
+    pos = np.array([0, 40, 7, -1, 300, 90, 33, 60, 12, 410, 15, 150] + [5, 260, 31] * 12, np.int32)
+    q_lens = np.minimum(rng.integers(1, few + 1, pos.size), few).astype(np.int32)
+    q_lens[:3] = few, 1, 0
+    q_lens[6], q_lens[7] = -1, q_len + 1
+    if many:
+        q_lens[4], q_lens[10] = q_len, few + 1
+    B, nblk = pos.size, (410 + q_len + bs - 1) // bs
+    kv = rng.standard_normal((2, B, nblk * bs, hkv, d), dtype=np.float32)
+    tables = rng.permutation(B * nblk).astype(np.int32).reshape(B, nblk)
+    paged = np.zeros((2, B * nblk, bs, hkv, d), np.float32)
+    for s in range(B):
+        paged[:, tables[s]] = kv[:, s].reshape(2, nblk, bs, hkv, d)
+    q = rng.standard_normal((B, q_len, hq, d), dtype=np.float32)
+    max_pos = 1 << 16
+    if ring:
+        rings = np.zeros((2, B, ring, hkv, d), np.float32)
+        slots = rng.permutation(B).astype(np.int32).reshape(B, 1)
+        for s in range(B):
+            for t in range(max(0, pos[s] + max(q_lens[s], 0) - ring), pos[s] + max(q_lens[s], 0)):
+                rings[:, slots[s, 0], t % ring] = kv[:, s, t]
+        p = make_params(LayerSpec(hq, hkv, d, window, F32, ring), bs, B, 0.0625)
+        got = _call("pkv_verify", p, q, rings[0], rings[1], slots, pos, q_lens, max_pos)
+    else:
+        p = make_params(LayerSpec(hq, hkv, d, window, F32), bs, B * nblk, 0.0625)
+        got = _call("pkv_verify", p, q, paged[0], paged[1], tables, pos, q_lens, max_pos)
+    for s in range(B):
+        n = int(q_lens[s])
+        if n < 0 or n > q_len:
+            assert np.all(np.isnan(got[s])), s
+            continue
+        assert np.all(got[s, n:] == 0), s  # rows past the count are not written
+        if n == 0 or pos[s] < 0:
+            assert np.all(got[s] == 0), s
+            continue
+        args = (n, hq, hkv, d, bs, window)
+        qs, ts, ps = q[s:s + 1, :n].copy(), tables[s:s + 1], pos[s:s + 1]
+        parity.check(got[s:s + 1, :n],
+                     O.attend(qs, paged[0].ravel(), paged[1].ravel(), ts, np.array([nblk], np.int32), ps, *args,
+                              scale=0.0625),
+                     O.attend_f64(qs, paged[0].ravel(), paged[1].ravel(), ts, ps, *args, scale=0.0625), what=f"{s}")
+
+
 @pytest.mark.parametrize("hq,hkv,d,q_len", [(16, 8, 256, 5), (16, 2, 512, 4)])
 @pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan])
 def test_rows_masked_values_not_finite(gpu, hq, hkv, d, q_len, value):
