@@ -101,3 +101,28 @@ def test_prefill_rows_outside_the_range(gpu, batch, bs, window, pos, n):
     lib.call("pkv_prefill", None, ctypes.byref(p), q.ptr, k.ptr, dv.ptr, dt.ptr, stride, dp.ptr, off.ptr, n, batch,
              1000, out.ptr)
     assert np.allclose(out.numpy(), 1.0, atol=1e-6)  # equal weights of rows of ones
+
+
+@pytest.mark.parametrize("n,pos", [(40, 900), (333, 900)], ids=["16-rows", "32-rows"])
+def test_prefill_split_precision(gpu, n, pos):
+    # Q, K and V are bf16 and exact; P enters as P_hi + P_lo, off by at most 2^-16 of p, and
+    # fp32 sums add less. The keys' errors are independent, so the output's relative error
+    # (2-norm) stays below 2^-16; without P_lo it would be about 3e-3 (P_hi truncates).
+    print(f"[prefill split] precision, {n} queries over {pos}", flush=True)
+    rng = np.random.default_rng(n)
+    hq, hkv, d, bs = 16, 8, 256, 16
+    nb = (pos + n + bs - 1) // bs
+    p = make_params(LayerSpec(hq, hkv, d, kv_dtype=BF16), bs, nb, 0.0625)
+    tables = rng.permutation(nb).astype(np.int32).reshape(1, nb)
+    q, k, v = (O.to_bf16(rng.standard_normal(s, dtype=np.float32)) for s in ((n, hq, d), (nb * bs * hkv * d,),
+                                                                            (nb * bs * hkv * d,)))
+    dq, dk, dv, dt, dp, off = (hip.DeviceArray.from_numpy(x) for x in (
+        q, k, v, tables, np.array([pos], np.int32), np.array([0, n], np.int32)))
+    out = hip.DeviceArray((n, hq, d), np.float32)
+    lib.call("pkv_prefill", None, ctypes.byref(p), dq.ptr, dk.ptr, dv.ptr, dt.ptr, nb, dp.ptr, off.ptr, n, 1,
+             pos + n - 1, out.ptr)
+    exact = O.attend_f64(O.bf16_to_f32(q)[None], O.bf16_to_f32(k), O.bf16_to_f32(v), tables, np.array([pos], np.int32),
+                         n, hq, hkv, d, bs, 0, scale=0.0625)[0]
+    err = np.linalg.norm(out.numpy() - exact) / np.linalg.norm(exact)
+    print(f"[prefill split] relative error {err:.2e}", flush=True)
+    assert err <= 2.0 ** -16

@@ -2,7 +2,8 @@
 against the oracle: row tiles (9, 16, 17, 32 rows, and one query group past 32), piece and
 batch edges (contexts 0 .. 33 and long ones, one sequence cut into many pieces), windows
 that open inside a batch, ring pools, and values that are not finite in keys some rows mask.
-Tolerances: tests/parity.py (sums in double, so 1e-5 against float64)."""
+Tolerances: tests/parity.py (sums in double, so 1e-5 against float64). Beside them the bf16 form
+for 9..16 rows: values that are not finite, precision, and pieces of one batch."""
 import ctypes
 
 import numpy as np
@@ -198,3 +199,34 @@ def test_bf16_wide_values_not_finite(gpu, hq, hkv, q_len, value):
             k1[tables[s, 1], 4][:, dim], k2[tables[s, 1], 4][:, dim] = low, inf
         a, b = (_call("pkv_attend", p, q, x, v, tables, pos) for x in (k1, k2))
         assert np.all(np.isfinite(b)) and np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("hq,hkv,q_len", [(16, 8, 5), (16, 16, 16)])
+def test_bf16_wide_precision(gpu, hq, hkv, q_len):
+    # Q and P enter as three bf16 parts, which are exact, so only fp32 roundings are left: about
+    # 24 in a score of size ~1 behind the scale, those of exp2 and of its argument, and the sums,
+    # 2^-24 of their size each and independent: 4e-7 to 6e-7 of the output (2-norm). 2e-6 leaves
+    # that four times; two parts of Q alone (off by 2^-17 of every element) give 4e-6.
+    print(f"[rows] bf16 wide precision {hq}q/{hkv}kv q_len {q_len}", flush=True)
+    rng = np.random.default_rng(q_len)
+    d, bs, pos = 256, 16, np.array([600, 1500, 45, 3000], np.int32)
+    nblk = (3000 + q_len + bs - 1) // bs
+    tables = rng.permutation(4 * nblk).astype(np.int32).reshape(4, nblk)
+    k, v = (O.to_bf16(rng.standard_normal((4 * nblk, bs, hkv, d), dtype=np.float32)) for _ in range(2))
+    q = rng.standard_normal((4, q_len, hq, d), dtype=np.float32)
+    p = make_params(LayerSpec(hq, hkv, d, 0, BF16), bs, 4 * nblk, 0.0625)
+    got = _call("pkv_attend", p, q, k, v, tables, pos)
+    exact = O.attend_f64(q, O.bf16_to_f32(k).ravel(), O.bf16_to_f32(v).ravel(), tables, pos, q_len, hq, hkv, d, bs, 0,
+                         scale=0.0625)
+    err = np.linalg.norm(got - exact) / np.linalg.norm(exact)
+    print(f"[rows] relative error {err:.2e}", flush=True)
+    assert err <= 2e-6
+
+
+@pytest.mark.parametrize("q_len", [4, 5], ids=["8-rows", "10-rows"])
+def test_bf16_pieces_of_one_batch(gpu, q_len):
+    # A workgroup's pieces of a single batch of keys follow one another with nothing to exchange
+    # between its waves; the next piece's Q must not reach LDS before every wave has read this one's.
+    print(f"[rows] bf16, 300 sequences of 1..12 keys, q_len {q_len}", flush=True)
+    rng = np.random.default_rng(q_len)
+    _batched_case(rng, 300, q_len, rng.integers(0, 12, 300), 16, 8, 256, 16, 0, BF16, 0.0625)
