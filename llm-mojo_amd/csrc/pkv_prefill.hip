@@ -241,7 +241,8 @@ __global__ __launch_bounds__(kNT) void prefill_kernel(PrefillArgs a) {
     // step before the copies that use it; a copy's address is that block's first row
     // (scalar) plus a per-lane offset that is the same for every tile. Keys outside
     // [k_lo, k_hi] (and tiles past the last) read rows of a valid block and are masked (their
-    // V rows zeroed, clean_v) or never read; a bad entry reads block 0 (the whole range was checked up front).
+    // V rows zeroed, clean_v) or never read; a bad entry reads block 0 (the whole range was
+    // checked up front).
     // K: lane i loads the global chunk that belongs at 16-byte position i % 32 of its row,
     // i.e. chunk (i % 32) ^ (key & 15). V: LDS position p of key row k holds global chunk
     // 2 * ((p / 2) ^ (k & 15)) + p % 2 (the 32-byte chunk swizzle).
@@ -579,8 +580,9 @@ __global__ __launch_bounds__(kNT) void prefill_kernel(PrefillArgs a) {
 // 4 grp + e % 4, P_hi for e < 4 and P_lo above, against V's operand of those keys given twice.
 // The row max is looked for across the lane groups only when a score passes the lazy
 // reference, the row sum only at the end.
-// One sequence of 333 tokens over 3001 cached ones (16q/8kv/256): 114 us in 48 workgroups of
-// 128 rows -> 62 us in 168 of 32; 64 tokens over 3000: 102 -> 41 us in 64 of 16. What bounds
+// One sequence of 333 tokens over 3001 cached ones (16q/8kv/256), back to back: 114 us in 48
+// workgroups of 128 rows -> 63 us in 168 of 32 (68 us in the trace of a step whose append has
+// just run); 64 tokens over 3000: 102 -> 41 us in 64 of 16. What bounds
 // it: every workgroup copies all its keys into LDS (128 KiB per round of 128 keys, 2048 cycles
 // at 64 B a cycle); a round takes about 3300 cycles with one tile and 4700 with two.
 template <int G, int RT>
@@ -651,7 +653,8 @@ __global__ __launch_bounds__(kNT) void prefill_split_kernel(PrefillArgs a) {
     // holds.
     // The lane's chunk of K in pair j is that of pair 0 with the bits of 2j flipped (the swizzle),
     // V's likewise. These and the operand addresses below are formed from an opaque copy of the
-    // lane where they are used: kept in registers they would spill beside Q and O of two tiles.
+    // lane where they are used: kept in registers they would spill beside Q and O of two tiles
+    // (which leave 248 of 256 registers used).
     auto opaque_lane = [&]() -> uint32_t {
         uint32_t x = lane;
         asm volatile("" : "+v"(x));

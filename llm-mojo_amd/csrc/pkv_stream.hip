@@ -478,8 +478,10 @@ __device__ inline KeySplit key_split(int total, int nwg) {
 }
 
 // Units of split work per key of a sequence with qc queries in this launch: what a key
-// costs stream_rows_kernel in matrix work and loads, by its 16-row tiles (one tile is bound
-// by its loads, two and three by the matrix cores).
+// costs stream_rows_kernel in loads and in matrix work, which grows with its 16-row tiles (one
+// or two). 16 sequences of 512..4096 keys at 16/2/512, 1..4 queries each: 119.5 us unweighted,
+// 99.9 with 1 + 2 tiles (97.8 with the tiles alone, 101.3 with 1 + tiles); 64 of 100..3000 keys
+// 304.9, 261.2 (270.3, 266.0). Sequences of one tile take the same time with any of them.
 __device__ inline int row_units(const StreamArgs& a, int qc) {
     return a.weighted ? 1 + 2 * ((a.G * qc + 15) >> 4) : 1;
 }
@@ -2403,7 +2405,7 @@ __global__ __launch_bounds__(kMaxWaves * kSW, 2) void stream_verify_kernel(Strea
 // accumulator, so O^T takes the same registers and nothing is folded. The keys' bytes bound it
 // (5.3 TB/s in the trace), so one pass instead of two halves the time of the second group, and
 // the third part costs nothing: 16 sequences of 512..4096 keys, 1..5 tokens at G = 2,
-// 60.5 + 4.7 (8 rows) + 20.6 + 5.3 us (2 rows) -> 62 + 5.0 us; error against
+// 60.5 + 4.7 (8 rows) + 20.6 + 5.3 us (2 rows) -> 63 + 5.0 us; error against
 // 64 bits 5.0e-6 -> 5.4e-7.
 // LDS per wave: K and V of 16 tokens, rows of 512 bytes; K's 16-byte chunk c of token r
 // sits at c ^ r and V's 32-byte chunk c at c ^ r, so the operand reads land on distinct
@@ -3225,8 +3227,8 @@ __global__ __launch_bounds__(merge_threads<D>()) void stream_merge_kernel(Stream
 // the plan, the (m, l) and the o of the first 32 pieces are requested together, later pieces
 // 64 at a time, where one thread per dim walks them eight at a time: one sequence of 8000 keys
 // at head_dim 512 in 512 pieces 38.8 -> 14.2 us (fp32), 35.4 -> 11.8 us (bf16), four of 4000
-// keys in 128 pieces each 14.5 -> 8.2 us. With a few pieces per sequence the smaller
-// workgroups only repeat the plan and the weights (LSA's ~9 pieces: 7.2 -> 8.6 us).
+// keys in 128 pieces each 14.5 -> 8.2 us. With many sequences of a few pieces the smaller
+// workgroups only repeat the plan and the weights (32 LSA lists of ~9 pieces: 7.2 -> 8.6 us).
 constexpr int kMergeNT = 256;
 constexpr int kMergeDims = 128;  // dims per workgroup
 template <int D, typename Acc>
@@ -3358,9 +3360,13 @@ __global__ __launch_bounds__(kMergeNT) void stream_merge_many_kernel(StreamArgs 
 
 // ---- host -------------------------------------------------------------------------
 
-// The merge of a launch of a.nwg workgroups along the keys. A sequence has about
-// a.nwg / batch pieces; from 32 on they are combined by stream_merge_many_kernel (128 pieces
-// 14.5 -> 8.2 us; at 16 the two take the same, 10.6 and 10.3 us).
+// The merge of a launch of a.nwg workgroups along the keys. A sequence has at most about
+// a.nwg / batch pieces (fewer where its keys end first, kPerMin to a piece); where that is 32 or
+// more they are combined by stream_merge_many_kernel (128 pieces 14.5 -> 8.2 us; at 16 the two
+// take the same, 10.6 and 10.3 us). With so few sequences it is also the faster one, or even,
+// where their keys leave fewer pieces: attention and merge of one sequence of 16 / 256 keys at
+// 16/8/256 10.5 -> 10.0 / 11.1 -> 10.4 us, eight at 16/2/512 17.3 -> 17.3 / 22.7 -> 22.3 us, LSA lists
+// of one / eight sequences 22.0 -> 19.9 / 24.3 -> 23.6 us.
 template <int D, typename Acc>
 void launch_merge(const StreamArgs& a, bool fused, hipStream_t st) {
     const int rows = a.batch + (fused ? 1 : 0);
@@ -3599,6 +3605,8 @@ int32_t launch_bf16_mfma(StreamArgs a, hipStream_t st) {
 }
 
 // fp32 pools with 9..32 query rows per kv head: stream_rows_kernel, grid (nwg, Hkv).
+// Lead-in in units of split work: 16 / 64 / 192 units on 16 sequences of 512..4096 keys at 16/2/512
+// with 1..5 queries 141.3 / 136.6 / 133.9 us, at 16/8/256 130.3 / 127.9 / 126.0 us.
 #ifndef PKV_LEAD_ROWS
 #define PKV_LEAD_ROWS 64
 #endif
@@ -3628,8 +3636,9 @@ int32_t launch_rows_kernel(StreamArgs a, hipStream_t st) {
     a.nwg = slots / a.Hkv > 0 ? slots / a.Hkv : 1;
     if (a.nwg > a.nwg_cap) a.nwg = a.nwg_cap;
     if (a.nwg > 1) a.nwg &= ~1;  // whole pairs (key_split)
-    // the weighted units of the split must fit an int
-    a.weighted = (int64_t)a.batch * (((int64_t)a.max_pos + 1) * 7 + PKV_LEAD_ROWS) <= INT32_MAX ? 1 : 0;
+    // the weighted units of the split (at most kRowUnits per key) must fit an int
+    constexpr int kRowUnits = 1 + 2 * ((kRowsMax + 15) / 16);
+    a.weighted = (int64_t)a.batch * (((int64_t)a.max_pos + 1) * kRowUnits + PKV_LEAD_ROWS) + kMaxSlots <= INT32_MAX ? 1 : 0;
     a.lead = PKV_LEAD_ROWS;
     hipLaunchKernelGGL(kernel, dim3(a.nwg, a.Hkv), dim3(kMaxWaves * kSW), lds, st, a);
     if (hipGetLastError() != hipSuccess)
@@ -3771,8 +3780,8 @@ int32_t stream_attend(const pkv_params* p, const float* q, const void* k_pool,
     if (stream_vector_lds(batch, nr != nullptr) > kStreamLdsMax)
         return fail(PKV_ERR_UNSUPPORTED, "stream path: batch too large for the kernel's LDS");
     const bool bf16 = p->kv_dtype == PKV_DTYPE_BF16;
-    // Queries in groups of at most 8 query rows per kv head, one launch pair each; the
-    // launches share the workspace in stream order.
+    // Queries in groups, one launch pair each; the launches share the workspace in stream order.
+    // A group has at most 8 query rows per kv head, or:
     // fp32 pools: from 9 rows on, groups of up to kRowsMax rows, each one pass over the keys
     // (10 rows 84 -> 72 us, 32 rows 251 -> 119 us against groups of 8; a remainder of up to 8
     // rows keeps the 8-row kernels, which waste no matrix rows).
